@@ -598,16 +598,14 @@ int rmsd_fit_to_ref(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frames*
   if (use_mass) {
     wpad = (double*)scratch(ctx, "fit.mass", sizeof(double) * ldr, &st);
     if (!wpad) return st;
-    HIP_TRY(ctx, hipMemsetAsync(wpad, 0, sizeof(double) * ldr, ctx->stream));
-    HIP_TRY(ctx, hipMemcpyAsync(wpad, frames->mass, sizeof(double) * n, hipMemcpyDeviceToDevice,
-                                ctx->stream));
   }
   const FrameSetDev F = to_dev(*frames);
   const FrameSetDev R = to_dev(*ref);
   ctx->marks = 0;
   mark(ctx, 0);
-  HIP_TRY(ctx, rmsd_launch_ref_prep(R, ref_frame, use_mass ? ref->mass : nullptr, wpad, fit ? 1 : 0,
-                                    refbuf, ref_trans, consts, ctx->stream));
+  HIP_TRY(ctx, rmsd_launch_ref_prep(R, ref_frame, use_mass ? ref->mass : nullptr,
+                                    use_mass ? frames->mass : nullptr, fit ? 1 : 0, refbuf,
+                                    ref_trans, consts, wpad, ctx->stream));
   if (!fit) {
     NofitArgs a;
     a.fs = F;
@@ -1006,7 +1004,7 @@ int rmsd_avgcorr(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frames* re
     if (!consts) return st;
     HIP_TRY(ctx, rmsd_launch_ref_prep(to_dev(*ref), ref_frame, use_mass ? ref->mass : nullptr,
                                       use_mass ? frames->mass : nullptr, 1, refbuf,
-                                      refbuf + 3 * ldr, consts, ctx->stream));
+                                      refbuf + 3 * ldr, consts, nullptr, ctx->stream));
   }
   if (method == RMSD_AVGCORR_RUNNING) {
     AvgCorrArgs a;
@@ -1182,9 +1180,6 @@ int rmsd_symm(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frames* ref, 
   if (use_mass) {
     wpad = (double*)scratch(ctx, "symm.mass", sizeof(double) * ldr, &st);
     if (!wpad) return st;
-    HIP_TRY(ctx, hipMemsetAsync(wpad, 0, sizeof(double) * ldr, ctx->stream));
-    HIP_TRY(ctx, hipMemcpyAsync(wpad, frames->mass, sizeof(double) * n, hipMemcpyDeviceToDevice,
-                                ctx->stream));
   }
   int* gmap = (int*)scratch(ctx, "symm.gmap", sizeof(int) * (size_t)(nf * std::max(S, 1)), &st);
   if (!gmap) return st;
@@ -1199,8 +1194,9 @@ int rmsd_symm(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frames* ref, 
   const FrameSetDev F = to_dev(*frames);
   ctx->marks = 0;
   mark(ctx, 0);
-  HIP_TRY(ctx, rmsd_launch_ref_prep(to_dev(*ref), ref_frame, use_mass ? ref->mass : nullptr, wpad,
-                                    fit ? 1 : 0, refbuf, ref_trans, consts, ctx->stream));
+  HIP_TRY(ctx, rmsd_launch_ref_prep(to_dev(*ref), ref_frame, use_mass ? ref->mass : nullptr,
+                                    use_mass ? frames->mass : nullptr, fit ? 1 : 0, refbuf,
+                                    ref_trans, consts, wpad, ctx->stream));
   double* U0 = nullptr;
   double* t0 = nullptr;
   double* moments = nullptr;

@@ -34,9 +34,6 @@ int rmsd_fit_backward(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frame
   if (use_mass) {
     wpad = (double*)scratch(ctx, "fit.mass", sizeof(double) * ldr, &st);
     if (!wpad) return st;
-    HIP_TRY(ctx, hipMemsetAsync(wpad, 0, sizeof(double) * ldr, ctx->stream));
-    HIP_TRY(ctx, hipMemcpyAsync(wpad, frames->mass, sizeof(double) * n, hipMemcpyDeviceToDevice,
-                                ctx->stream));
   }
   double* moments = (double*)scratch(ctx, "fit.moments", sizeof(double) * 16 * nf, &st);
   if (!moments) return st;
@@ -48,8 +45,9 @@ int rmsd_fit_backward(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frame
   const FrameSetDev R = to_dev(*ref);
   // Recompute the per-frame rotations (moments + QCP) rather than keeping
   // them from the forward call.
-  HIP_TRY(ctx, rmsd_launch_ref_prep(R, ref_frame, use_mass ? ref->mass : nullptr, wpad, 1, refbuf,
-                                    ref_trans, consts, ctx->stream));
+  HIP_TRY(ctx, rmsd_launch_ref_prep(R, ref_frame, use_mass ? ref->mass : nullptr,
+                                    use_mass ? frames->mass : nullptr, 1, refbuf, ref_trans, consts,
+                                    wpad, ctx->stream));
   FitArgs fa;
   fa.fs = F;
   fa.mass = wpad;

@@ -32,14 +32,6 @@ constexpr int MAX_DEVICES = 64;
 std::mutex g_mu;
 void* g_ptr[MAX_DEVICES] = {};
 
-// Padded target masses: w[k] = mass[k] for k < n, 0 up to ldr (the fit
-// kernels read whole quads).  A kernel instead of a memset + copy, so the
-// sequence is also valid under stream capture.
-__global__ void k_pad_mass(double* w, const double* mass, int n, int ldr) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < ldr) w[k] = k < n ? mass[k] : 0.0;
-}
-
 // Layout of one call in the scratch array, each piece starting on a 256-byte
 // boundary as the context's own scratch buffers do: reference SoA + its
 // translation (3 ldr + 8), constants (8), padded masses (ldr), moments (16 per
@@ -133,14 +125,9 @@ int rmsd_fit_to_ref_noalloc(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd
   double* xform = base + lay.xform;
   const FrameSetDev F = to_dev(*frames);
   const FrameSetDev R = to_dev(*ref);
-  if (use_mass) {
-    hipLaunchKernelGGL(k_pad_mass, dim3((ldr + 255) / 256), dim3(256), 0, ctx->stream, wpad,
-                       frames->mass, n, ldr);
-    HIP_TRY(ctx, hipGetLastError());
-  }
   HIP_TRY(ctx, rmsd_launch_ref_prep(R, ref_frame, use_mass ? ref->mass : nullptr,
-                                    use_mass ? wpad : nullptr, fit ? 1 : 0, refbuf, ref_trans,
-                                    consts, ctx->stream));
+                                    use_mass ? frames->mass : nullptr, fit ? 1 : 0, refbuf,
+                                    ref_trans, consts, wpad, ctx->stream));
   if (!fit) {
     NofitArgs a;
     a.fs = F;

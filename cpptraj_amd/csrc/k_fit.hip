@@ -39,19 +39,65 @@ __device__ __forceinline__ float fcoord(const FrameSetDev& fs, int64_t f, int k,
 // ---- reference ---------------------------------------------------------------
 // ref_out: SoA [3][ldr] FP64 (ldr = nsel rounded up to 4, zero padded).
 // consts: [0..2] sum w y, [3] sum w |y|^2, [4] W = sum w (sequential sum, so
-// that it rounds exactly as the reference's running total).
-__global__ __launch_bounds__(FIT_THREADS) void k_ref_prep(FrameSetDev fs, int f, const double* rmass,
+// that it rounds exactly as the reference's running total).  wpad (with tmass):
+// the masses padded with zeros to ldr, for the kernels that read whole quads.
+//
+// Two workgroups: the sequential sum is a chain of nsel dependent additions, so
+// workgroup 1 runs it from LDS (masses staged by all its threads) beside the
+// centring in workgroup 0.  One thread summing straight from memory, behind the
+// centring, took 140 us for 2,000 masses and 212 us for 3,000 (a load's latency
+// per few masses); now 13 and 19 us.  Workgroup 0 has 1,024 threads: it is
+// alone on the chip and bound by the latency of its trips over the atoms.
+constexpr int REF_THREADS = 1024;
+constexpr int REF_STAGE = 2048;  // masses per LDS stage
+
+__device__ __forceinline__ void mass_chain(const double* m, int n, int ldr, double* wpad,
+                                           double* stage, double* W) {
+  double s = 0.0;
+  for (int k0 = 0; k0 < ldr; k0 += REF_STAGE) {
+    const int c = ldr - k0 < REF_STAGE ? ldr - k0 : REF_STAGE;
+    for (int k = threadIdx.x; k < c; k += blockDim.x) {
+      const double v = k0 + k < n ? m[k0 + k] : 0.0;
+      stage[k] = v;
+      if (wpad) wpad[k0 + k] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      const int real = n - k0 < c ? n - k0 : c;  // the padding is not added
+      int k = 0;
+      for (; k + 16 <= real; k += 16) {
+        double v[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) v[e] = stage[k + e];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) s += v[e];
+      }
+      for (; k < real; ++k) s += stage[k];
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) *W = s;
+}
+
+__global__ __launch_bounds__(REF_THREADS) void k_ref_prep(FrameSetDev fs, int f, const double* rmass,
                                                           const double* tmass, int center, int ldr,
                                                           double* ref_out, double* ref_trans,
-                                                          double* consts) {
-  __shared__ double red[8 * (FIT_THREADS / 64)];
+                                                          double* consts, double* wpad) {
+  __shared__ double sm[REF_STAGE];
+  if (blockIdx.x == 1) {
+    mass_chain(tmass, fs.nsel, ldr, wpad, sm, consts + 4);
+    return;
+  }
+  double* red = sm;  // 4 sums per wave
   double v[4] = {0, 0, 0, 0};
   if (center) {
     for (int k = threadIdx.x; k < fs.nsel; k += blockDim.x) {
       const double m = rmass ? rmass[k] : 1.0;
-      v[0] += (double)fcoord(fs, f, k, 0) * m;
-      v[1] += (double)fcoord(fs, f, k, 1) * m;
-      v[2] += (double)fcoord(fs, f, k, 2) * m;
+      float p[3];
+      load_atom(fs, f, k, p);
+      v[0] += (double)p[0] * m;
+      v[1] += (double)p[1] * m;
+      v[2] += (double)p[2] * m;
       v[3] += m;
     }
     rmsd_dev::block_sum<4>(v, red);
@@ -69,9 +115,11 @@ __global__ __launch_bounds__(FIT_THREADS) void k_ref_prep(FrameSetDev fs, int f,
   for (int k = threadIdx.x; k < ldr; k += blockDim.x) {
     double y[3] = {0, 0, 0};
     if (k < fs.nsel) {
-      y[0] = (double)fcoord(fs, f, k, 0) - cen[0];
-      y[1] = (double)fcoord(fs, f, k, 1) - cen[1];
-      y[2] = (double)fcoord(fs, f, k, 2) - cen[2];
+      float p[3];
+      load_atom(fs, f, k, p);
+      y[0] = (double)p[0] - cen[0];
+      y[1] = (double)p[1] - cen[1];
+      y[2] = (double)p[2] - cen[2];
       const double w = tmass ? tmass[k] : 1.0;
       h[0] += w * y[0];
       h[1] += w * y[1];
@@ -88,13 +136,7 @@ __global__ __launch_bounds__(FIT_THREADS) void k_ref_prep(FrameSetDev fs, int f,
     consts[1] = h[1];
     consts[2] = h[2];
     consts[3] = h[3];
-    double W = 0.0;
-    if (tmass) {
-      for (int k = 0; k < fs.nsel; ++k) W += tmass[k];
-    } else {
-      W = (double)fs.nsel;
-    }
-    consts[4] = W;
+    if (!tmass) consts[4] = (double)fs.nsel;
     ref_trans[0] = cen[0];
     ref_trans[1] = cen[1];
     ref_trans[2] = cen[2];
@@ -721,10 +763,10 @@ __global__ __launch_bounds__(FIT_THREADS) void k_apply(ApplyArgs a, int mode) {
 
 hipError_t rmsd_launch_ref_prep(const FrameSetDev& fs, int f, const double* rmass,
                                 const double* tmass, int center, double* ref_out,
-                                double* ref_trans, double* consts, hipStream_t s) {
+                                double* ref_trans, double* consts, double* wpad, hipStream_t s) {
   const int ldr = (fs.nsel + 3) & ~3;
-  hipLaunchKernelGGL(k_ref_prep, dim3(1), dim3(FIT_THREADS), 0, s, fs, f, rmass, tmass, center, ldr,
-                     ref_out, ref_trans, consts);
+  hipLaunchKernelGGL(k_ref_prep, dim3(tmass ? 2 : 1), dim3(REF_THREADS), 0, s, fs, f, rmass, tmass,
+                     center, ldr, ref_out, ref_trans, consts, wpad);
   return hipGetLastError();
 }
 

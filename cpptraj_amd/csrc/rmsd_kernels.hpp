@@ -427,9 +427,11 @@ hipError_t rmsd_launch_nofit_frames(const NofitArgs& a, const double* consts, do
 hipError_t rmsd_launch_apply(const ApplyArgs& a, int mode, hipStream_t s);
 hipError_t rmsd_launch_rotate_ucell(const double* U, int64_t nframes, double* ucell,
                                     hipStream_t s);
+// Centred reference, its constants and, with target masses (tmass: nsel, as
+// the caller holds them), their copy zero-padded to whole quads (wpad, may be null).
 hipError_t rmsd_launch_ref_prep(const FrameSetDev& fs, int f, const double* rmass,
                                 const double* tmass, int center, double* ref_out,
-                                double* ref_trans, double* consts, hipStream_t s);
+                                double* ref_trans, double* consts, double* wpad, hipStream_t s);
 
 // Gradients (k_grad.hip).
 hipError_t rmsd_launch_fit_grad(const FrameSetDev& fs, const double* mass, const double* ref,

@@ -154,3 +154,17 @@ def test_fit_aos_padded_stride_tail(oracle, ctx, use_mass):
     assert_rmsd_close(r, r_o, X3.reshape(F, -1))
     assert np.abs(U - U_o).max() <= 1e-9
     assert np.abs(tv - tv_o).max() <= 1e-9
+
+
+@pytest.mark.parametrize("n", [2, 3, 16, 17, 1023, 2047, 2048, 2049, 4101])
+def test_total_mass_stages(oracle, ctx, n):
+    """The reference's sequential mass sum in stages of 2,048 masses and steps
+    of 16: atom counts at their edges.  Without fit RMSD^2 = sum / W, so the
+    relative error of W shows undiminished (1e-12: the parallel sum's)."""
+    import cpptraj_amd as ca
+    X = synth.noisy(6, 5, n, 1.0).reshape(5, -1)
+    m = synth.masses(np.random.default_rng(n), n)
+    r_o, _, _, _ = oracle_fit(oracle, X, None, m, True, fit=False)
+    r, _, _ = ca.rmsd_fit(dev(X), None, 0, mass=dev(m), fit=False, use_mass=True, modify="nomod",
+                          ctx=ctx)
+    np.testing.assert_allclose(r.cpu().numpy(), r_o, rtol=1e-12, atol=0)
