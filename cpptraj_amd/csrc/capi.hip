@@ -178,6 +178,109 @@ BoundCoef rmsd_bound_coef(int prec, int KB) {
   return k;
 }
 
+// Whether writing `frames` in place could change frame ref_frame of `ref` (a
+// reference frame list lives on the device: assumed to).
+static bool shares_frame(const rmsd_frames& frames, const rmsd_frames& ref, int ref_frame) {
+  if (ref.fidx) return true;
+  auto extent = [](const rmsd_frames& f) {
+    return f.ld ? 2 * f.ld + (int64_t)f.natom : 3 * (int64_t)f.natom;
+  };
+  const float* f0 = frames.xyz;
+  const float* f1 = f0 + (int64_t)(frames.nframes - 1) * frames.stride + extent(frames);
+  const float* r0 = ref.xyz + (int64_t)ref_frame * ref.stride;
+  return r0 < f1 && f0 < r0 + extent(ref);
+}
+
+FitPlan fit_plan(const rmsd_frames& frames, const rmsd_frames& ref, int ref_frame, int fit,
+                 int modify) {
+  FitPlan p;
+  p.fit = fit != 0;
+  p.fused = p.fit && rmsd_fit_fused_fits(frames.natom, frames.nsel, frames.nframes, modify);
+  // Workgroups that prepare the reference read it while others rewrite frames.
+  p.inref = p.fused && rmsd_fit_inref_fits(frames.natom, frames.nsel, frames.nframes, modify) &&
+            (modify == RMSD_MODIFY_NONE || !shares_frame(frames, ref, ref_frame));
+  return p;
+}
+
+int fit_enqueue(rmsd_ctx* c, const FitPlan& plan, const FitBuffers& b, const rmsd_frames& frames,
+                const rmsd_frames& ref, int ref_frame, int use_mass, int modify, double* rmsd,
+                double* U, double* tvec) {
+  const FrameSetDev F = to_dev(frames);
+  const FrameSetDev R = to_dev(ref);
+  const double* tmass = use_mass ? frames.mass : nullptr;
+  const double* rmass = use_mass ? ref.mass : nullptr;
+  double* ref_trans = b.ref ? b.ref + 3 * round_up(frames.nsel, 4) : nullptr;
+  double* wpad = use_mass ? b.wpad : nullptr;
+  mark(c, 0);
+  if (plan.reference())
+    HIP_TRY(c, rmsd_launch_ref_prep(R, ref_frame, rmass, tmass, plan.fit ? 1 : 0, b.ref, ref_trans,
+                                    b.consts, wpad, c->stream));
+  mark(c, 1);
+  if (!plan.fit) {
+    NofitArgs a;
+    a.fs = F;
+    a.mass = wpad;
+    a.ref = b.ref;
+    HIP_TRY(c, rmsd_launch_nofit_frames(a, b.consts, rmsd, c->stream));
+    mark(c, 2);
+    mark(c, 3);
+    return RMSD_OK;
+  }
+  if (plan.fused) {
+    FitFusedArgs a;
+    a.fs = F;
+    a.natom = frames.natom;
+    a.mode = modify == RMSD_MODIFY_ROT_TRANS ? 1 : (modify == RMSD_MODIFY_TRANS ? 2 : 0);
+    a.mass = plan.inref ? tmass : wpad;
+    a.ref = b.ref;
+    a.consts = b.consts;
+    a.ref_trans = ref_trans;
+    a.R = R;
+    a.ref_frame = ref_frame;
+    a.rmass = rmass;
+    a.clamp = 1;
+    a.rmsd = rmsd;
+    a.U = U;
+    a.tvec = tvec;
+    HIP_TRY(c, rmsd_launch_fit_fused(a, c->stream));
+    mark(c, 2);
+    mark(c, 3);
+    return RMSD_OK;
+  }
+  FitArgs fa;
+  fa.fs = F;
+  fa.mass = wpad;
+  fa.ref = b.ref;
+  fa.consts = b.consts;
+  fa.moments = b.moments;
+  HIP_TRY(c, rmsd_launch_fit_moments(fa, c->stream));
+  mark(c, 2);
+  SolveArgs sa;
+  sa.moments = b.moments;
+  sa.consts = b.consts;
+  sa.ref_trans = ref_trans;
+  sa.nframes = frames.nframes;
+  sa.fit = 1;
+  sa.clamp = 1;
+  sa.rmsd = rmsd;
+  sa.U = U;
+  sa.tvec = tvec;
+  sa.xform = b.xform;
+  HIP_TRY(c, rmsd_launch_fit_solve(sa, c->stream));
+  if (modify != RMSD_MODIFY_NONE) {
+    ApplyArgs ap;
+    ap.xyz = const_cast<float*>(frames.xyz);
+    ap.stride = frames.stride;
+    ap.ld = frames.ld;
+    ap.natom = frames.natom;
+    ap.nframes = frames.nframes;
+    ap.xform = b.xform;
+    HIP_TRY(c, rmsd_launch_apply(ap, modify == RMSD_MODIFY_ROT_TRANS ? 1 : 2, c->stream));
+  }
+  mark(c, 3);
+  return RMSD_OK;
+}
+
 }  // namespace rmsd_capi
 
 using namespace rmsd_capi;
@@ -586,77 +689,30 @@ int rmsd_fit_to_ref(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frames*
   if (!rmsd && frames->nframes > 0) return fail(ctx, RMSD_ERR_ARG, "rmsd is NULL");
   if (frames->nframes == 0) return RMSD_OK;
   HIP_TRY(ctx, hipSetDevice(ctx->device));
-  const int n = frames->nsel;
-  const int ldr = (int)round_up(n, 4);
+  const FitPlan plan = fit_plan(*frames, *ref, ref_frame, fit, modify);
+  const int64_t ldr = round_up(frames->nsel, 4);
   const int64_t nf = frames->nframes;
-  double* refbuf = (double*)scratch(ctx, "fit.ref", sizeof(double) * (3 * ldr + 8), &st);
-  if (!refbuf) return st;
-  double* ref_trans = refbuf + 3 * ldr;
-  double* consts = (double*)scratch(ctx, "fit.consts", sizeof(double) * 8, &st);
-  if (!consts) return st;
-  double* wpad = nullptr;
-  if (use_mass) {
-    wpad = (double*)scratch(ctx, "fit.mass", sizeof(double) * ldr, &st);
-    if (!wpad) return st;
+  FitBuffers b;
+  if (plan.reference()) {
+    b.ref = (double*)scratch(ctx, "fit.ref", sizeof(double) * (3 * ldr + 8), &st);
+    if (!b.ref) return st;
+    b.consts = (double*)scratch(ctx, "fit.consts", sizeof(double) * 8, &st);
+    if (!b.consts) return st;
+    if (use_mass) {
+      b.wpad = (double*)scratch(ctx, "fit.mass", sizeof(double) * ldr, &st);
+      if (!b.wpad) return st;
+    }
   }
-  const FrameSetDev F = to_dev(*frames);
-  const FrameSetDev R = to_dev(*ref);
+  if (plan.moments()) {
+    b.moments = (double*)scratch(ctx, "fit.moments", sizeof(double) * 16 * nf, &st);
+    if (!b.moments) return st;
+  }
+  if (plan.xform(modify)) {
+    b.xform = (double*)scratch(ctx, "fit.xform", sizeof(double) * 15 * nf, &st);
+    if (!b.xform) return st;
+  }
   ctx->marks = 0;
-  mark(ctx, 0);
-  HIP_TRY(ctx, rmsd_launch_ref_prep(R, ref_frame, use_mass ? ref->mass : nullptr,
-                                    use_mass ? frames->mass : nullptr, fit ? 1 : 0, refbuf,
-                                    ref_trans, consts, wpad, ctx->stream));
-  if (!fit) {
-    NofitArgs a;
-    a.fs = F;
-    a.mass = wpad;
-    a.ref = refbuf;
-    mark(ctx, 1);
-    HIP_TRY(ctx, rmsd_launch_nofit_frames(a, consts, rmsd, ctx->stream));
-    mark(ctx, 2);
-    mark(ctx, 3);
-    return RMSD_OK;
-  }
-  double* moments = (double*)scratch(ctx, "fit.moments", sizeof(double) * 16 * nf, &st);
-  if (!moments) return st;
-  double* xform = nullptr;
-  if (modify != RMSD_MODIFY_NONE) {
-    xform = (double*)scratch(ctx, "fit.xform", sizeof(double) * 15 * nf, &st);
-    if (!xform) return st;
-  }
-  FitArgs fa;
-  fa.fs = F;
-  fa.mass = wpad;
-  fa.ref = refbuf;
-  fa.consts = consts;
-  fa.moments = moments;
-  mark(ctx, 1);
-  HIP_TRY(ctx, rmsd_launch_fit_moments(fa, ctx->stream));
-  mark(ctx, 2);
-  SolveArgs sa;
-  sa.moments = moments;
-  sa.consts = consts;
-  sa.ref_trans = ref_trans;
-  sa.nframes = (int)nf;
-  sa.fit = 1;
-  sa.clamp = 1;
-  sa.rmsd = rmsd;
-  sa.U = U;
-  sa.tvec = tvec;
-  sa.xform = xform;
-  HIP_TRY(ctx, rmsd_launch_fit_solve(sa, ctx->stream));
-  if (modify != RMSD_MODIFY_NONE) {
-    ApplyArgs ap;
-    ap.xyz = const_cast<float*>(frames->xyz);
-    ap.stride = frames->stride;
-    ap.ld = frames->ld;
-    ap.natom = frames->natom;
-    ap.nframes = frames->nframes;
-    ap.xform = xform;
-    HIP_TRY(ctx, rmsd_launch_apply(ap, modify == RMSD_MODIFY_ROT_TRANS ? 1 : 2, ctx->stream));
-  }
-  mark(ctx, 3);
-  return RMSD_OK;
+  return fit_enqueue(ctx, plan, b, *frames, *ref, ref_frame, use_mass, modify, rmsd, U, tvec);
 }
 
 int rmsd_fit_pairs(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frames* refs, int fit,

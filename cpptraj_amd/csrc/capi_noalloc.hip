@@ -117,55 +117,16 @@ int rmsd_fit_to_ref_noalloc(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd
                     "); split the frames into smaller calls");
   HIP_TRY(ctx, hipSetDevice(ctx->device));
   double* base = static_cast<double*>(ctx->noalloc);
-  double* refbuf = base + lay.ref;
-  double* ref_trans = refbuf + 3 * ldr;
-  double* consts = base + lay.consts;
-  double* wpad = base + lay.wpad;
-  double* moments = base + lay.moments;
-  double* xform = base + lay.xform;
-  const FrameSetDev F = to_dev(*frames);
-  const FrameSetDev R = to_dev(*ref);
-  HIP_TRY(ctx, rmsd_launch_ref_prep(R, ref_frame, use_mass ? ref->mass : nullptr,
-                                    use_mass ? frames->mass : nullptr, fit ? 1 : 0, refbuf,
-                                    ref_trans, consts, wpad, ctx->stream));
-  if (!fit) {
-    NofitArgs a;
-    a.fs = F;
-    a.mass = use_mass ? wpad : nullptr;
-    a.ref = refbuf;
-    HIP_TRY(ctx, rmsd_launch_nofit_frames(a, consts, rmsd, ctx->stream));
-    return RMSD_OK;
+  const FitPlan plan = fit_plan(*frames, *ref, ref_frame, fit, modify);
+  FitBuffers b;
+  if (plan.reference()) {
+    b.ref = base + lay.ref;
+    b.consts = base + lay.consts;
+    b.wpad = base + lay.wpad;
   }
-  FitArgs fa;
-  fa.fs = F;
-  fa.mass = use_mass ? wpad : nullptr;
-  fa.ref = refbuf;
-  fa.consts = consts;
-  fa.moments = moments;
-  HIP_TRY(ctx, rmsd_launch_fit_moments(fa, ctx->stream));
-  SolveArgs sa;
-  sa.moments = moments;
-  sa.consts = consts;
-  sa.ref_trans = ref_trans;
-  sa.nframes = (int)nf;
-  sa.fit = 1;
-  sa.clamp = 1;
-  sa.rmsd = rmsd;
-  sa.U = U;
-  sa.tvec = tvec;
-  sa.xform = modify != RMSD_MODIFY_NONE ? xform : nullptr;
-  HIP_TRY(ctx, rmsd_launch_fit_solve(sa, ctx->stream));
-  if (modify != RMSD_MODIFY_NONE) {
-    ApplyArgs ap;
-    ap.xyz = const_cast<float*>(frames->xyz);
-    ap.stride = frames->stride;
-    ap.ld = frames->ld;
-    ap.natom = frames->natom;
-    ap.nframes = frames->nframes;
-    ap.xform = xform;
-    HIP_TRY(ctx, rmsd_launch_apply(ap, modify == RMSD_MODIFY_ROT_TRANS ? 1 : 2, ctx->stream));
-  }
-  return RMSD_OK;
+  if (plan.moments()) b.moments = base + lay.moments;
+  if (plan.xform(modify)) b.xform = base + lay.xform;
+  return fit_enqueue(ctx, plan, b, *frames, *ref, ref_frame, use_mass, modify, rmsd, U, tvec);
 }
 
 }  // extern "C"

@@ -21,10 +21,11 @@
 // molecule's extent only, not its absolute position.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
-#include "rmsd_device.hpp"
-#include "rmsd_kernels.hpp"
+#include "fit_device.hpp"
 
 namespace {
+
+using namespace fit_dev;
 
 constexpr int FIT_THREADS = 256;
 
@@ -46,8 +47,9 @@ __device__ __forceinline__ float fcoord(const FrameSetDev& fs, int64_t f, int k,
 // workgroup 1 runs it from LDS (masses staged by all its threads) beside the
 // centring in workgroup 0.  One thread summing straight from memory, behind the
 // centring, took 140 us for 2,000 masses and 212 us for 3,000 (a load's latency
-// per few masses); now 13 and 19 us.  Workgroup 0 has 1,024 threads: it is
-// alone on the chip and bound by the latency of its trips over the atoms.
+// per few masses); now 13 and 19 us.  Workgroup 0 is
+// alone on the chip and bound by the latency of its trips over the atoms, hence
+// 1,024 threads for more than two trips of 256.
 constexpr int REF_THREADS = 1024;
 constexpr int REF_STAGE = 2048;  // masses per LDS stage
 
@@ -144,24 +146,6 @@ __global__ __launch_bounds__(REF_THREADS) void k_ref_prep(FrameSetDev fs, int f,
 }
 
 // ---- moments -----------------------------------------------------------------
-template <bool WEIGHTED>
-__device__ __forceinline__ void accum(double (&v)[13], double x0, double x1, double x2, double w,
-                                      double y0, double y1, double y2) {
-  double wx0 = x0, wx1 = x1, wx2 = x2;
-  if (WEIGHTED) {
-    wx0 = w * x0;
-    wx1 = w * x1;
-    wx2 = w * x2;
-  }
-  v[0] += wx0;
-  v[1] += wx1;
-  v[2] += wx2;
-  v[3] += wx0 * y0; v[4] += wx0 * y1; v[5] += wx0 * y2;
-  v[6] += wx1 * y0; v[7] += wx1 * y1; v[8] += wx1 * y2;
-  v[9] += wx2 * y0; v[10] += wx2 * y1; v[11] += wx2 * y2;
-  v[12] += wx0 * x0 + wx1 * x1 + wx2 * x2;
-}
-
 // Vector path: SoA rows, no selection, 16-byte aligned rows.
 template <bool WEIGHTED>
 __global__ __launch_bounds__(FIT_THREADS) void k_fit_moments_soa4(FitArgs a, int ldr) {
@@ -237,14 +221,12 @@ __global__ __launch_bounds__(FIT_THREADS) void k_fit_moments_any(FitArgs a, int 
 // f = wave id, + total waves, ...  A frame's 16 sums are combined with the
 // butterfly of wave_reduce16, so there is no block barrier per frame; HBM and
 // the vector memory pipe carry the frames only (12 B per atom), LDS serves the
-// reference (24 or 32 B per atom).  VEC: SoA rows, no selection, 16-byte
-// aligned rows, four atoms per lane per step.  Also stores the per-frame shift.
+// reference (24 or 32 B per atom).  Also stores the per-frame shift.  Frames
+// with a selection, one atom per lane and step; k_fit_moments_aos4 and
+// k_fit_moments_wave2 take the others.
 constexpr int WAVE_FIT_THREADS = 1024;
-// Frames a wave streams side by side on the VEC path (1 or 2; two measured
-// 5 % faster on 1e6 x 3000 frames).
-constexpr int kFitFramesPerWave = 2;
 
-template <bool VEC, bool WEIGHTED>
+template <bool WEIGHTED>
 __global__ __launch_bounds__(WAVE_FIT_THREADS) void k_fit_moments_wave(FitArgs a, int ldr,
                                                                        double* shift) {
   extern __shared__ double sref[];  // [3][ldr] centred reference, then [ldr] weights
@@ -255,43 +237,19 @@ __global__ __launch_bounds__(WAVE_FIT_THREADS) void k_fit_moments_wave(FitArgs a
   __syncthreads();
   const int lane = threadIdx.x & 63;
   const int64_t nw = (int64_t)gridDim.x * (blockDim.x >> 6);
-  const int64_t ld = a.fs.ld;
   const double* Y0 = sref;
   const double* Y1 = sref + ldr;
   const double* Y2 = sref + 2 * ldr;
   const double* Wt = sref + 3 * ldr;
   for (int64_t f = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
        f < a.fs.nframes; f += nw) {
-    const float* fr = a.fs.xyz + frame_of(a.fs, f) * a.fs.stride;
     const double s0 = fcoord(a.fs, f, 0, 0), s1 = fcoord(a.fs, f, 0, 1), s2 = fcoord(a.fs, f, 0, 2);
     double v[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) v[i] = 0.0;
     double (&m)[13] = *reinterpret_cast<double(*)[13]>(v);
-    int k0 = 0;
-    if (VEC) {
-      const int n4 = n >> 2;
-      const f32x4* X = reinterpret_cast<const f32x4*>(fr);
-      const f32x4* Y = reinterpret_cast<const f32x4*>(fr + ld);
-      const f32x4* Z = reinterpret_cast<const f32x4*>(fr + 2 * ld);
 #pragma unroll 4
-      for (int q = lane; q < n4; q += 64) {
-        const f32x4 x = __builtin_nontemporal_load(X + q);
-        const f32x4 y = __builtin_nontemporal_load(Y + q);
-        const f32x4 z = __builtin_nontemporal_load(Z + q);
-        const int k = 4 * q;
-        accum<WEIGHTED>(m, x.x - s0, y.x - s1, z.x - s2, WEIGHTED ? Wt[k] : 1.0, Y0[k], Y1[k], Y2[k]);
-        accum<WEIGHTED>(m, x.y - s0, y.y - s1, z.y - s2, WEIGHTED ? Wt[k + 1] : 1.0, Y0[k + 1],
-                        Y1[k + 1], Y2[k + 1]);
-        accum<WEIGHTED>(m, x.z - s0, y.z - s1, z.z - s2, WEIGHTED ? Wt[k + 2] : 1.0, Y0[k + 2],
-                        Y1[k + 2], Y2[k + 2]);
-        accum<WEIGHTED>(m, x.w - s0, y.w - s1, z.w - s2, WEIGHTED ? Wt[k + 3] : 1.0, Y0[k + 3],
-                        Y1[k + 3], Y2[k + 3]);
-      }
-      k0 = 4 * n4;
-    }
-#pragma unroll 4
-    for (int k = k0 + lane; k < n; k += 64) {
+    for (int k = lane; k < n; k += 64) {
       float p[3];
       load_atom(a.fs, f, k, p);
       accum<WEIGHTED>(m, (double)p[0] - s0, (double)p[1] - s1, (double)p[2] - s2,
@@ -308,14 +266,14 @@ __global__ __launch_bounds__(WAVE_FIT_THREADS) void k_fit_moments_wave(FitArgs a
   }
 }
 
-// Two frames per wave (VEC layout only): the frames f and f + nwaves stream
+// Two frames per wave (SoA rows): the frames f and f + nwaves stream
 // side by side through the same atom blocks, so a wave keeps twice the loads
 // in flight and one LDS read of the reference serves both frames.
 constexpr int WAVE2_FIT_THREADS = 512;
 
 // One frame per wave for AoS frames without a selection (cpptraj's own
 // layout): a lane takes four consecutive atoms, twelve floats, as three
-// 16-byte loads, so consecutive lanes read consecutive 48 bytes.  The
+// 16-byte loads (any dword address serves, so any base and stride do), so consecutive lanes read consecutive 48 bytes.  The
 // reference sits in LDS as twelve arrays over atom quads (component d of atom
 // 4q + i at [(3i + d) Q + q]), masses as four, so each LDS read is contiguous
 // across the wave; a lane reading Y_d[4q + i] from the plain [3][ldr] table
@@ -354,12 +312,12 @@ __global__ __launch_bounds__(WAVE_FIT_THREADS) void k_fit_moments_aos4(FitArgs a
 #pragma unroll
     for (int i = 0; i < 16; ++i) v[i] = 0.0;
     double (&m)[13] = *reinterpret_cast<double(*)[13]>(v);
-    const f32x4* V = reinterpret_cast<const f32x4*>(fr);
+    const f32x4_a4* V = reinterpret_cast<const f32x4_a4*>(fr);
 #pragma unroll 1  // as in k_fit_moments_wave2 (here 1-2 % faster than by two)
     for (int q = lane; q < Q; q += 64) {
-      const f32x4 p0 = V[3 * q];
-      const f32x4 p1 = V[3 * q + 1];
-      const f32x4 p2 = V[3 * q + 2];
+      const f32x4_a4 p0 = V[3 * q];
+      const f32x4_a4 p1 = V[3 * q + 1];
+      const f32x4_a4 p2 = V[3 * q + 2];
       accum<WEIGHTED>(m, p0.x - s0, p0.y - s1, p0.z - s2, WEIGHTED ? Wq[q] : 1.0, Yq[q],
                       Yq[Q + q], Yq[2 * Q + q]);
       accum<WEIGHTED>(m, p0.w - s0, p1.x - s1, p1.y - s2, WEIGHTED ? Wq[Q + q] : 1.0,
@@ -415,22 +373,22 @@ __global__ __launch_bounds__(WAVE2_FIT_THREADS) void k_fit_moments_wave2(FitArgs
     for (int i = 0; i < 16; ++i) va[i] = vb[i] = 0.0;
     double (&ma)[13] = *reinterpret_cast<double(*)[13]>(va);
     double (&mb)[13] = *reinterpret_cast<double(*)[13]>(vb);
-    const f32x4* XA = reinterpret_cast<const f32x4*>(fa);
-    const f32x4* YA = reinterpret_cast<const f32x4*>(fa + ld);
-    const f32x4* ZA = reinterpret_cast<const f32x4*>(fa + 2 * ld);
-    const f32x4* XB = reinterpret_cast<const f32x4*>(fb);
-    const f32x4* YB = reinterpret_cast<const f32x4*>(fb + ld);
-    const f32x4* ZB = reinterpret_cast<const f32x4*>(fb + 2 * ld);
+    const f32x4_a4* XA = reinterpret_cast<const f32x4_a4*>(fa);
+    const f32x4_a4* YA = reinterpret_cast<const f32x4_a4*>(fa + ld);
+    const f32x4_a4* ZA = reinterpret_cast<const f32x4_a4*>(fa + 2 * ld);
+    const f32x4_a4* XB = reinterpret_cast<const f32x4_a4*>(fb);
+    const f32x4_a4* YB = reinterpret_cast<const f32x4_a4*>(fb + ld);
+    const f32x4_a4* ZB = reinterpret_cast<const f32x4_a4*>(fb + 2 * ld);
 // One 16-byte step per loop trip: unrolling by two measured 8 % slower
     // (5.36-5.41 vs 5.82-5.86 TB/s on 500,000 x 3,000; 241 vs 167 registers).
 #pragma unroll 1
     for (int q = lane; q < n4; q += 64) {
-      const f32x4 xa = __builtin_nontemporal_load(XA + q);
-      const f32x4 ya = __builtin_nontemporal_load(YA + q);
-      const f32x4 za = __builtin_nontemporal_load(ZA + q);
-      const f32x4 xb = __builtin_nontemporal_load(XB + q);
-      const f32x4 yb = __builtin_nontemporal_load(YB + q);
-      const f32x4 zb = __builtin_nontemporal_load(ZB + q);
+      const f32x4_a4 xa = __builtin_nontemporal_load(XA + q);
+      const f32x4_a4 ya = __builtin_nontemporal_load(YA + q);
+      const f32x4_a4 za = __builtin_nontemporal_load(ZA + q);
+      const f32x4_a4 xb = __builtin_nontemporal_load(XB + q);
+      const f32x4_a4 yb = __builtin_nontemporal_load(YB + q);
+      const f32x4_a4 zb = __builtin_nontemporal_load(ZB + q);
       const int k = 4 * q;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -488,31 +446,9 @@ __global__ void k_fit_shift(FrameSetDev fs, double* shift) {
 __global__ void k_fit_solve(SolveArgs a, const double* shift) {
   const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (f >= a.nframes) return;
-  const double* m = a.moments + 13 * f;
-  const double* K = a.consts;
-  const double W = K[4];
-  double U[9] = {1, 0, 0, 0, 1, 0, 0, 0, 1};
-  double t1[3] = {0, 0, 0};
-  double r;
-  if (W < RMSD_SMALL) {
-    r = -1.0;
-  } else {
-    // centroid in shifted coordinates, then the centred moments
-    const double c0 = m[0] / W, c1 = m[1] / W, c2 = m[2] / W;
-    double R[9];
-    R[0] = m[3] - c0 * K[0]; R[1] = m[4] - c0 * K[1]; R[2] = m[5] - c0 * K[2];
-    R[3] = m[6] - c1 * K[0]; R[4] = m[7] - c1 * K[1]; R[5] = m[8] - c1 * K[2];
-    R[6] = m[9] - c2 * K[0]; R[7] = m[10] - c2 * K[1]; R[8] = m[11] - c2 * K[2];
-    const double sx = m[12] - W * (c0 * c0 + c1 * c1 + c2 * c2);
-    const double E0 = 0.5 * (sx + K[3]);
-    const rmsd_dev::QcpCoef co = rmsd_dev::qcp_coefficients(R);
-    const double lam = rmsd_dev::qcp_lambda(co, E0);
-    r = rmsd_dev::rmsd_from_lambda(E0, lam, W, a.clamp);
-    rmsd_dev::qcp_rotation(R, lam, U);
-    t1[0] = -(c0 + shift[3 * f]);
-    t1[1] = -(c1 + shift[3 * f + 1]);
-    t1[2] = -(c2 + shift[3 * f + 2]);
-  }
+  double U[9], t1[3];
+  const double r = solve(a.moments + 13 * f, a.consts, shift[3 * f], shift[3 * f + 1],
+                         shift[3 * f + 2], a.clamp, U, t1);
   a.rmsd[f] = r;
   if (a.U)
     for (int k = 0; k < 9; ++k) a.U[9 * f + k] = U[k];
@@ -728,7 +664,6 @@ __global__ __launch_bounds__(FIT_THREADS) void k_nofit_frames(NofitArgs a, int l
 // atoms are all natom or the list atoms[0..natoms-1] (Trans_Rot_Trans with an
 // AtomMask, as Action_Align's 'move' uses it).
 __global__ __launch_bounds__(FIT_THREADS) void k_apply(ApplyArgs a, int mode) {
-#pragma clang fp contract(off)
   const int64_t f = blockIdx.x;
   double X[15];
   if (a.xform) {
@@ -738,24 +673,22 @@ __global__ __launch_bounds__(FIT_THREADS) void k_apply(ApplyArgs a, int mode) {
     for (int k = 0; k < 6; ++k) X[9 + k] = a.tvec[6 * f + k];
   }
   float* fr = a.xyz + f * a.stride;  // all stored frames, in order
+  // Every atom: quads in 16-byte accesses, then the last natom mod 4.
+  const int n4 = a.atoms ? 0 : a.natom >> 2;
+  for (int q = threadIdx.x; q < n4; q += blockDim.x) {
+    float x[4], y[4], z[4];
+    load_step(fr, a.ld, q, x, y, z);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) move_atom(X, mode, x[e], y[e], z[e]);
+    store_step(fr, a.ld, q, x, y, z);
+  }
   const int nmove = a.atoms ? a.natoms : a.natom;
-  for (int i = threadIdx.x; i < nmove; i += blockDim.x) {
+  for (int i = 4 * n4 + threadIdx.x; i < nmove; i += blockDim.x) {
     const int k = a.atoms ? a.atoms[i] : i;
     float* px = a.ld ? fr + k : fr + 3 * k;
     float* py = a.ld ? fr + a.ld + k : fr + 3 * k + 1;
     float* pz = a.ld ? fr + 2 * a.ld + k : fr + 3 * k + 2;
-    if (mode == 1) {
-      const double x = (double)*px + X[9];
-      const double y = (double)*py + X[10];
-      const double z = (double)*pz + X[11];
-      *px = (float)(x * X[0] + y * X[1] + z * X[2] + X[12]);
-      *py = (float)(x * X[3] + y * X[4] + z * X[5] + X[13]);
-      *pz = (float)(x * X[6] + y * X[7] + z * X[8] + X[14]);
-    } else {
-      *px = (float)((double)*px + (X[9] + X[12]));
-      *py = (float)((double)*py + (X[10] + X[13]));
-      *pz = (float)((double)*pz + (X[11] + X[14]));
-    }
+    move_atom(X, mode, *px, *py, *pz);
   }
 }
 
@@ -765,7 +698,8 @@ hipError_t rmsd_launch_ref_prep(const FrameSetDev& fs, int f, const double* rmas
                                 const double* tmass, int center, double* ref_out,
                                 double* ref_trans, double* consts, double* wpad, hipStream_t s) {
   const int ldr = (fs.nsel + 3) & ~3;
-  hipLaunchKernelGGL(k_ref_prep, dim3(tmass ? 2 : 1), dim3(REF_THREADS), 0, s, fs, f, rmass, tmass,
+  const int threads = fs.nsel <= 512 ? 256 : REF_THREADS;
+  hipLaunchKernelGGL(k_ref_prep, dim3(tmass ? 2 : 1), dim3(threads), 0, s, fs, f, rmass, tmass,
                      center, ldr, ref_out, ref_trans, consts, wpad);
   return hipGetLastError();
 }
@@ -809,22 +743,23 @@ hipError_t rmsd_launch_fit_moments(const FitArgs& a, hipStream_t s) {
   if (nf == 0) return hipSuccess;
   const bool vec = a.fs.sel == nullptr && a.fs.ld > 0 && (a.fs.ld % 4) == 0 &&
                    (a.fs.stride % 4) == 0 && ((uintptr_t)a.fs.xyz % 16) == 0;
-  const bool aos4 = a.fs.sel == nullptr && a.fs.ld == 0 && (a.fs.stride % 4) == 0 &&
-                    ((uintptr_t)a.fs.xyz % 16) == 0;
+  // Quads of atoms, unless they would leave half of a wave's lanes idle.
+  const bool quads = a.fs.sel == nullptr && a.fs.nsel > FIT_SINGLE_ATOMS;
+  const bool aos4 = quads && a.fs.ld == 0, soa = quads && a.fs.ld > 0;
   const bool w = a.mass != nullptr;
   // Wave-per-frame path whenever the reference fits in LDS (up to 5120
   // weighted / 6826 unweighted atoms); one-block-per-frame kernels otherwise.
   const size_t lds = wave_fit_lds(ldr, w);
-  if (lds && a.variant != 1) {
+  if (lds) {
     int dev = 0, ncu = 256;
     hipGetDevice(&dev);
     hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
     const int64_t waves = WAVE_FIT_THREADS / 64;
     const int64_t want = (nf + waves - 1) / waves;
     // Blocks loop over frames, so the grid must not exceed what is resident.
-#define RMSD_FIT_WAVE(V, W)                                                                   \
+#define RMSD_FIT_WAVE(W)                                                                   \
   {                                                                                          \
-    const void* fn = reinterpret_cast<const void*>(&k_fit_moments_wave<V, W>);               \
+    const void* fn = reinterpret_cast<const void*>(&k_fit_moments_wave<W>);               \
     hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
     if (e != hipSuccess) return e;                                                           \
     int bpc = 1;                                                                             \
@@ -832,7 +767,7 @@ hipError_t rmsd_launch_fit_moments(const FitArgs& a, hipStream_t s) {
     if (e != hipSuccess) return e;                                                           \
     if (bpc < 1) bpc = 1;                                                                    \
     const int grid = (int)(want < (int64_t)ncu * bpc ? want : (int64_t)ncu * bpc);           \
-    hipLaunchKernelGGL((k_fit_moments_wave<V, W>), dim3(grid), dim3(WAVE_FIT_THREADS), lds, s, a, \
+    hipLaunchKernelGGL((k_fit_moments_wave<W>), dim3(grid), dim3(WAVE_FIT_THREADS), lds, s, a, \
                        ldr, shift);                                                          \
   }
 #define RMSD_FIT_WAVE2(W)                                                                     \
@@ -862,14 +797,12 @@ hipError_t rmsd_launch_fit_moments(const FitArgs& a, hipStream_t s) {
     hipLaunchKernelGGL((k_fit_moments_aos4<W>), dim3(grid), dim3(WAVE_FIT_THREADS), lds, s, a, \
                        ldr, shift);                                                          \
   }
-    if (vec && kFitFramesPerWave == 2) {
+    if (soa) {
       if (w) RMSD_FIT_WAVE2(true) else RMSD_FIT_WAVE2(false)
     } else if (aos4) {
       if (w) RMSD_FIT_AOS4(true) else RMSD_FIT_AOS4(false)
-    } else if (vec) {
-      if (w) RMSD_FIT_WAVE(true, true) else RMSD_FIT_WAVE(true, false)
     } else {
-      if (w) RMSD_FIT_WAVE(false, true) else RMSD_FIT_WAVE(false, false)
+      if (w) RMSD_FIT_WAVE(true) else RMSD_FIT_WAVE(false)
     }
 #undef RMSD_FIT_WAVE
 #undef RMSD_FIT_WAVE2

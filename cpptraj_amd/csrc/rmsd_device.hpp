@@ -247,6 +247,7 @@ __device__ __forceinline__ int qcp_rotation(const double* S, double lam, double*
   double q4 = -a21 * m3243 + a22 * m3143 - a23 * m3142;
   double qq = q1 * q1 + q2 * q2 + q3 * q3 + q4 * q4;
   const double eps = 1e-6;
+  int ok = 1;
   if (qq < eps) {
     q1 = a12 * m3344 - a13 * m3244 + a14 * m3243;
     q2 = -a11 * m3344 + a13 * m3144 - a14 * m3143;
@@ -269,9 +270,11 @@ __device__ __forceinline__ int qcp_rotation(const double* S, double lam, double*
         q4 = -a31 * m1223 + a32 * m1123 - a33 * m1122;
         qq = q1 * q1 + q2 * q2 + q3 * q3 + q4 * q4;
         if (qq < eps) {
-          U[0] = U[4] = U[8] = 1.0;
-          U[1] = U[2] = U[3] = U[5] = U[6] = U[7] = 0.0;
-          return 0;
+          // the identity, as the quaternion (1, 0, 0, 0): one set of stores to
+          // U keeps it in registers
+          q1 = qq = 1.0;
+          q2 = q3 = q4 = 0.0;
+          ok = 0;
         }
       }
     }
@@ -294,7 +297,7 @@ __device__ __forceinline__ int qcp_rotation(const double* S, double lam, double*
   U[2] = 2 * (zx + wy);
   U[5] = 2 * (yz - wx);
   U[8] = w2 - x2 - y2 + z2;
-  return 1;
+  return ok;
 }
 
 // ---- reductions -----------------------------------------------------------

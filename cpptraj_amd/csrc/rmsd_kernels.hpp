@@ -235,7 +235,6 @@ struct FitArgs {
   const double* ref;     // centred reference, SoA [3][nsel] FP64
   const double* consts;  // [0..2] sum w y, [3] sum w |y|^2, [4] total weight
   double* moments;       // out: 13 per frame, then 3 per frame of shift
-  int variant = 0;       // 0: fastest fitting kernel, 1: one block per frame
 };
 
 struct SolveArgs {
@@ -250,6 +249,31 @@ struct SolveArgs {
   double* tvec;             // 6 per frame or null
   double* xform;            // 15 per frame (U, Trans, refTrans) for the coordinate update, or null
 };
+
+// Moments, solve and update of every frame in one launch (k_fit_fused.hip).
+struct FitFusedArgs {
+  FrameSetDev fs;          // frames (fitted atoms); rewritten in place when mode != 0
+  int natom;               // stored atoms per frame (moved by the update)
+  int mode;                // 0: none, 1: rotate + translate, 2: translate
+  const double* mass;      // weights of the fitted atoms (null: unit)
+  const double* ref;       // rmsd_launch_ref_prep's outputs, or ref null: every
+  const double* consts;    // workgroup prepares frame ref_frame of R itself
+  const double* ref_trans;
+  FrameSetDev R;
+  int ref_frame;
+  const double* rmass;     // centring masses of the reference (null: unit)
+  int clamp;
+  double* rmsd;
+  double* U;               // 9 per frame or null
+  double* tvec;            // 6 per frame or null
+};
+constexpr int FIT_SINGLE_ATOMS = 128;   // up to here a lane takes single atoms, beyond quads
+constexpr int FIT_MANY_FRAMES = 16384;  // from here a wave takes several small frames
+constexpr int FIT_FUSED_FRAMES = 1024;  // without update: more frames take the moment kernels
+constexpr int FIT_INREF_FRAMES = 512;   // more frames: the reference is prepared once, before
+bool rmsd_fit_fused_fits(int natom, int nsel, int nframes, int mode);
+bool rmsd_fit_inref_fits(int natom, int nsel, int nframes, int mode);
+hipError_t rmsd_launch_fit_fused(const FitFusedArgs& a, hipStream_t s);
 
 // Fit of target frame f of T to reference frame f of R, every f (k_fit.hip,
 // k_fit_pairs): the 'reftraj' and 'previous' reference modes of

@@ -168,3 +168,86 @@ def test_total_mass_stages(oracle, ctx, n):
     r, _, _ = ca.rmsd_fit(dev(X), None, 0, mass=dev(m), fit=False, use_mass=True, modify="nomod",
                           ctx=ctx)
     np.testing.assert_allclose(r.cpu().numpy(), r_o, rtol=1e-12, atol=0)
+
+
+@pytest.mark.parametrize("modify", ["nomod", "rottrans", "norotate"])
+@pytest.mark.parametrize("layout", ["aos", "soa", "sel"])
+@pytest.mark.parametrize("n", [1, 3, 5, 255, 256, 259, 513, 1024, 1031, 2051, 3075, 4097, 8195])
+def test_fit_in_registers_edges(oracle, ctx, n, layout, modify):
+    """Frames at the edges of the kernels that hold them in registers (threads
+    and quads per frame, the last atoms, frames beyond them), unaligned rows and
+    strides, against the oracle: RMSD, vectors and rewritten coordinates."""
+    import cpptraj_amd as ca
+    F = 5
+    X3 = synth.noisy(n, F + 1, n, 1.0)
+    X, R = X3[:F].reshape(F, -1), X3[F:]
+    sel = np.arange(0, n, 2, dtype=np.int32)[::-1].copy() if layout == "sel" else None
+    um = n % 2 == 1
+    k = n if sel is None else len(sel)
+    m = synth.masses(np.random.default_rng(n), k)
+    ref = R[0].astype(np.float64) if sel is None else R[0][sel].astype(np.float64)
+    rc, rt = oracle.center_on_origin(ref, m, um)
+    mod = {"nomod": 0, "rottrans": 1, "norotate": 2}[modify]
+    r_o, U_o, tv_o, fo = oracle.fit_frames(X, rc, rt, sel=sel, mass=m, fit=True, use_mass=um,
+                                           modify=mod, want_frames=True)
+    soa = layout == "soa"
+    Xd = dev(synth.to_soa(X3[:F], ld=n + 3)) if soa else dev(X)
+    Rd = dev(synth.to_soa(R, ld=n + 3)) if soa else dev(R.reshape(1, -1))
+    r, U, tv = ca.rmsd_fit(Xd, Rd, mask=None if sel is None else dev(sel), mass=dev(m),
+                           use_mass=um, modify=modify, save_matrices=True, save_vectors=True,
+                           soa=soa, natom=n, ctx=ctx)
+    if k == 2:
+        # A double root of the QCP quartic: sqrt(eps) from the oracle's Jacobi on
+        # every path.  The moment kernels' bits instead (a call of 4,100 frames).
+        rm, _, _ = ca.rmsd_fit(dev(np.tile(X, (820, 1))), dev(R.reshape(1, -1)), mask=dev(sel),
+                               mass=dev(m), use_mass=um, modify="nomod", ctx=ctx)
+        assert np.array_equal(r.cpu().numpy(), rm[:F].cpu().numpy())
+    else:
+        assert_rmsd_close(r.cpu().numpy(), r_o, X)
+    assert np.abs(tv.cpu().numpy() - tv_o).max() <= 1e-9
+    if k > 3:  # fewer atoms: the rotation is not unique
+        assert np.abs(U.cpu().numpy() - U_o).max() <= 1e-9
+        got = Xd.cpu().numpy()
+        if soa:
+            assert not got[:, :, n:].any()  # the rows' padding stays
+            got = np.transpose(got[:, :, :n], (0, 2, 1)).reshape(F, -1)
+        exp = fo if mod else X
+        ulp = np.spacing(np.abs(exp).astype(np.float32))
+        assert np.all(np.abs(got - exp) <= 2 * ulp + 1e-5 * (mod == 1) * (k < 8) + 1e-30)
+
+
+@pytest.mark.parametrize("layout", ["aos", "soa", "sel"])
+@pytest.mark.parametrize("n", [30, 331, 512, 1023])
+def test_fit_same_bits_for_any_frame_count(ctx, n, layout):
+    """A frame's results do not depend on how many frames the call has: the
+    reference prepared per workgroup, once before, or the moment kernels."""
+    import cpptraj_amd as ca
+    import torch
+    X3 = synth.noisy(n, 4200, n, 1.0)
+    m = synth.masses(np.random.default_rng(n), n)
+    sel = dev(np.arange(0, n, 3, dtype=np.int32)) if layout == "sel" else None
+    soa = layout == "soa"
+    X = dev(synth.to_soa(X3, ld=n + 1)) if soa else dev(X3.reshape(4200, -1))
+    R = X[7:8].clone()
+    k = n if sel is None else sel.numel()
+
+    def fit(F):
+        return ca.rmsd_fit(X[:F], R, mask=sel, mass=dev(m[:k]), use_mass=True, modify="nomod",
+                           save_matrices=True, save_vectors=True, soa=soa, natom=n, ctx=ctx)
+    full = fit(4200)
+    for F in (3, 600):
+        for a, b in zip(fit(F), full):
+            assert torch.equal(a, b[:F])
+
+
+def test_fit_reference_among_the_rewritten_frames(oracle, ctx):
+    """'first' with the update: frame 0 is the reference and is rewritten."""
+    import cpptraj_amd as ca
+    F, n = 40, 90
+    X = synth.noisy(11, F, n, 1.0).reshape(F, -1)
+    r_o, _, _, fo = oracle_fit(oracle, X, None, None, False, modify=1)
+    Xd = dev(X)
+    r, _, _ = ca.rmsd_fit(Xd, None, 0, ctx=ctx)
+    assert_rmsd_close(r.cpu().numpy(), r_o, X)
+    ulp = np.spacing(np.abs(fo).astype(np.float32))
+    assert np.all(np.abs(Xd.cpu().numpy() - fo) <= 2 * ulp + 1e-30)
