@@ -128,6 +128,9 @@ def _optional(L):
     if hasattr(L, "rmsd_fit_backward"):
         L.rmsd_fit_backward.argtypes = [P, FP, FP, C.c_int, C.c_int, P, P]
         L.rmsd_fit_backward.restype = C.c_int
+    if hasattr(L, "rmsd_fit_backward_f32"):
+        L.rmsd_fit_backward_f32.argtypes = [P, FP, FP, C.c_int, C.c_int, P, P]
+        L.rmsd_fit_backward_f32.restype = C.c_int
     if hasattr(L, "rmsd_pairwise_backward"):
         L.rmsd_pairwise_backward.argtypes = [P, FP, FP, C.c_int, P, P, P]
         L.rmsd_pairwise_backward.restype = C.c_int

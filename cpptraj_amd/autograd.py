@@ -6,8 +6,8 @@
   ``rmsd_pairwise_backward`` (rotations recomputed in FP64).
 
 Coordinates are float32 CUDA tensors of shape (F, n, 3) (the selected atoms,
-AoS).  Forward and backward run in the HIP library; the FP64 gradient is cast to
-the input dtype for autograd.
+AoS).  Forward and backward run in the HIP library; gradients are FP64, rounded
+to the input dtype for autograd.
 """
 from __future__ import annotations
 
@@ -26,6 +26,11 @@ def _ctx(dev) -> Context:
 
 def fit_backward(frames, ref, grad_rmsd, mass=None, use_mass=False, ctx: Context | None = None):
     """FP64 d(sum_f g_f RMSD_f)/d frames, shape (F, n, 3)."""
+    return _fit_backward(frames, ref, grad_rmsd, mass, use_mass, torch.float64, ctx)
+
+
+def _fit_backward(frames, ref, grad_rmsd, mass, use_mass, dtype, ctx=None):
+    """fit_backward, computed in FP64 and stored as `dtype` (float64 or float32)."""
     ctx = ctx or _ctx(frames.device)
     L = load_library()
     F, n = frames.shape[0], frames.shape[1]
@@ -33,10 +38,11 @@ def fit_backward(frames, ref, grad_rmsd, mass=None, use_mass=False, ctx: Context
     fc, rc = frames.contiguous(), ref.contiguous()
     d = frames_desc(fc, None, mass)
     r = frames_desc(rc, None, mass)
-    g = torch.empty((F, n, 3), dtype=torch.float64, device=frames.device)
+    g = torch.empty((F, n, 3), dtype=dtype, device=frames.device)
     gr = grad_rmsd.to(torch.float64).contiguous()
-    ctx.check(L.rmsd_fit_backward(ctx.handle, C.byref(d), C.byref(r), 0, int(use_mass),
-                                  C.c_void_p(gr.data_ptr()), C.c_void_p(g.data_ptr())))
+    fn = L.rmsd_fit_backward if dtype == torch.float64 else L.rmsd_fit_backward_f32
+    ctx.check(fn(ctx.handle, C.byref(d), C.byref(r), 0, int(use_mass), C.c_void_p(gr.data_ptr()),
+                 C.c_void_p(g.data_ptr())))
     return g
 
 
@@ -81,8 +87,8 @@ class RmsdToReference(torch.autograd.Function):
     @staticmethod
     def backward(fctx, g):
         frames, ref = fctx.saved_tensors
-        grad = fit_backward(frames, ref, g, fctx.mass, fctx.use_mass)
-        return grad.to(frames.dtype), None, None, None
+        grad = _fit_backward(frames, ref, g, fctx.mass, fctx.use_mass, frames.dtype)
+        return grad, None, None, None
 
 
 class PairwiseRmsd(torch.autograd.Function):

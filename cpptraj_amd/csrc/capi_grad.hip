@@ -5,10 +5,10 @@
 
 using namespace rmsd_capi;
 
-extern "C" {
+namespace {
 
-int rmsd_fit_backward(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frames* ref,
-                      int ref_frame, int use_mass, const double* grad_rmsd, double* grad_xyz) {
+int fit_backward(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frames* ref, int ref_frame,
+                 int use_mass, const double* grad_rmsd, void* grad_xyz, bool f32) {
   if (!ctx) return RMSD_ERR_ARG;
   int st;
   if ((st = check_frames(ctx, frames, "frames")) != RMSD_OK) return st;
@@ -25,15 +25,51 @@ int rmsd_fit_backward(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frame
   const int n = frames->nsel;
   const int ldr = (int)round_up(n, 4);
   const int64_t nf = frames->nframes;
-  double* refbuf = (double*)scratch(ctx, "fit.ref", sizeof(double) * (3 * ldr + 8), &st);
-  if (!refbuf) return st;
-  double* ref_trans = refbuf + 3 * ldr;
-  double* consts = (double*)scratch(ctx, "fit.consts", sizeof(double) * 8, &st);
-  if (!consts) return st;
+  const FrameSetDev F = to_dev(*frames);
+  const FrameSetDev R = to_dev(*ref);
+  const double* tmass = use_mass ? frames->mass : nullptr;
+  const double* rmass = use_mass ? ref->mass : nullptr;
+  // The rotations are recomputed (moments + QCP) rather than kept from the
+  // forward call; with the frame held in registers that reads nothing twice.
+  const bool fused = rmsd_fit_grad_fits(F);
+  const bool inref = fused && rmsd_fit_inref_fits(n, n, frames->nframes, 0);
+  double* refbuf = nullptr;
+  double* ref_trans = nullptr;
+  double* consts = nullptr;
   double* wpad = nullptr;
-  if (use_mass) {
-    wpad = (double*)scratch(ctx, "fit.mass", sizeof(double) * ldr, &st);
-    if (!wpad) return st;
+  if (!inref) {
+    refbuf = (double*)scratch(ctx, "fit.ref", sizeof(double) * (3 * ldr + 8), &st);
+    if (!refbuf) return st;
+    ref_trans = refbuf + 3 * ldr;
+    consts = (double*)scratch(ctx, "fit.consts", sizeof(double) * 8, &st);
+    if (!consts) return st;
+    if (use_mass) {
+      wpad = (double*)scratch(ctx, "fit.mass", sizeof(double) * ldr, &st);
+      if (!wpad) return st;
+    }
+    HIP_TRY(ctx, rmsd_launch_ref_prep(R, ref_frame, rmass, tmass, 1, refbuf, ref_trans, consts,
+                                      wpad, ctx->stream));
+  }
+  if (fused) {
+    FitFusedArgs a;
+    a.fs = F;
+    a.natom = n;
+    a.mode = 0;
+    a.mass = inref ? tmass : wpad;
+    a.ref = refbuf;
+    a.consts = consts;
+    a.ref_trans = ref_trans;
+    a.R = R;
+    a.ref_frame = ref_frame;
+    a.rmass = rmass;
+    a.clamp = 1;
+    a.rmsd = nullptr;
+    a.U = nullptr;
+    a.tvec = nullptr;
+    a.gout = grad_rmsd;
+    a.grad = grad_xyz;
+    HIP_TRY(ctx, rmsd_launch_fit_grad_fused(a, f32, ctx->stream));
+    return RMSD_OK;
   }
   double* moments = (double*)scratch(ctx, "fit.moments", sizeof(double) * 16 * nf, &st);
   if (!moments) return st;
@@ -41,13 +77,6 @@ int rmsd_fit_backward(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frame
   if (!xform) return st;
   double* rm = (double*)scratch(ctx, "fit.rmsd", sizeof(double) * nf, &st);
   if (!rm) return st;
-  const FrameSetDev F = to_dev(*frames);
-  const FrameSetDev R = to_dev(*ref);
-  // Recompute the per-frame rotations (moments + QCP) rather than keeping
-  // them from the forward call.
-  HIP_TRY(ctx, rmsd_launch_ref_prep(R, ref_frame, use_mass ? ref->mass : nullptr,
-                                    use_mass ? frames->mass : nullptr, 1, refbuf, ref_trans, consts,
-                                    wpad, ctx->stream));
   FitArgs fa;
   fa.fs = F;
   fa.mass = wpad;
@@ -67,9 +96,23 @@ int rmsd_fit_backward(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frame
   sa.tvec = nullptr;
   sa.xform = xform;
   HIP_TRY(ctx, rmsd_launch_fit_solve(sa, ctx->stream));
-  HIP_TRY(ctx, rmsd_launch_fit_grad(F, wpad, refbuf, xform, rm, grad_rmsd, consts, grad_xyz,
+  HIP_TRY(ctx, rmsd_launch_fit_grad(F, wpad, refbuf, xform, rm, grad_rmsd, consts, grad_xyz, f32,
                                     ctx->stream));
   return RMSD_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int rmsd_fit_backward(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frames* ref,
+                      int ref_frame, int use_mass, const double* grad_rmsd, double* grad_xyz) {
+  return fit_backward(ctx, frames, ref, ref_frame, use_mass, grad_rmsd, grad_xyz, false);
+}
+
+int rmsd_fit_backward_f32(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frames* ref,
+                          int ref_frame, int use_mass, const double* grad_rmsd, float* grad_xyz) {
+  return fit_backward(ctx, frames, ref, ref_frame, use_mass, grad_rmsd, grad_xyz, true);
 }
 
 int rmsd_pairwise_backward(rmsd_ctx* ctx, const rmsd_frames* A, const rmsd_frames* B,

@@ -61,7 +61,7 @@ __device__ __forceinline__ double solve(const double* m, const double* K, double
 
 // X = U (9), t1 (3), t2 (3).  mode 1: x' = U (x + t1) + t2
 // (Frame::Trans_Rot_Trans, in its operation order); mode 2: x' = x + (t1 + t2).
-__device__ __forceinline__ void move_atom(const double (&X)[15], int mode, float& px, float& py,
+__device__ __forceinline__ void move_atom(const double* X, int mode, float& px, float& py,
                                           float& pz) {
 #pragma clang fp contract(off)
   if (mode == 1) {

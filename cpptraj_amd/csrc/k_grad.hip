@@ -12,7 +12,8 @@
 // AoS [frame][atom][3].
 //
 //   k_fit_grad    streaming: frame-to-reference fit (rotations recomputed by
-//                 the moments + solve kernels of k_fit.hip, not stored)
+//                 the moments + solve kernels of k_fit.hip, not stored), for
+//                 frames with a selection or too large for k_fit_fused.hip
 //   k_center      per frame FP64 centred coordinates and E0 halves
 //   k_pair_rot    per 16 x 16 block of pairs (i, j): covariances on FP64
 //                 MFMA, then per pair QCP and rotation; stores c_ij = G_ij /
@@ -27,19 +28,19 @@
 namespace {
 
 // xform: 15 doubles per frame (U, t1 = -centroid, t2) from k_fit_solve.
+template <class G>
 __global__ __launch_bounds__(256) void k_fit_grad(FrameSetDev fs, const double* mass, const double* ref,
                                                   int ldr, const double* xform, const double* rmsd,
-                                                  const double* gout, const double* consts,
-                                                  double* grad) {
+                                                  const double* gout, const double* consts, G* grad) {
   const int64_t f = blockIdx.y;
   const double W = consts[4];
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= fs.nsel) return;
   const double* X = xform + 15 * f;
   const double r = rmsd[f];
-  double* g = grad + (f * fs.nsel + k) * 3;
+  G* g = grad + (f * fs.nsel + k) * 3;
   if (!(r > 1e-12) || W < RMSD_SMALL) {
-    g[0] = g[1] = g[2] = 0.0;
+    g[0] = g[1] = g[2] = G(0);
     return;
   }
   const double s = gout[f] * (mass ? mass[k] : 1.0) / (W * r);
@@ -53,9 +54,9 @@ __global__ __launch_bounds__(256) void k_fit_grad(FrameSetDev fs, const double* 
   const double u0 = X[0] * y0 + X[3] * y1 + X[6] * y2;
   const double u1 = X[1] * y0 + X[4] * y1 + X[7] * y2;
   const double u2 = X[2] * y0 + X[5] * y1 + X[8] * y2;
-  g[0] = s * (x0 - u0);
-  g[1] = s * (x1 - u1);
-  g[2] = s * (x2 - u2);
+  g[0] = (G)(s * (x0 - u0));
+  g[1] = (G)(s * (x1 - u1));
+  g[2] = (G)(s * (x2 - u2));
 }
 
 // Centred FP64 coordinates, SoA [F][3][n], and sum w |x~|^2 per frame.
@@ -312,11 +313,15 @@ __global__ __launch_bounds__(256) void k_grad_sum(const double* XA, const double
 
 hipError_t rmsd_launch_fit_grad(const FrameSetDev& fs, const double* mass, const double* ref,
                                 const double* xform, const double* rmsd, const double* gout,
-                                const double* consts, double* grad, hipStream_t s) {
+                                const double* consts, void* grad, bool f32, hipStream_t s) {
   const int ldr = (fs.nsel + 3) & ~3;
   dim3 grid((fs.nsel + 255) / 256, fs.nframes);
-  hipLaunchKernelGGL(k_fit_grad, grid, dim3(256), 0, s, fs, mass, ref, ldr, xform, rmsd, gout,
-                     consts, grad);
+  if (f32)
+    hipLaunchKernelGGL(k_fit_grad<float>, grid, dim3(256), 0, s, fs, mass, ref, ldr, xform, rmsd,
+                       gout, consts, static_cast<float*>(grad));
+  else
+    hipLaunchKernelGGL(k_fit_grad<double>, grid, dim3(256), 0, s, fs, mass, ref, ldr, xform, rmsd,
+                       gout, consts, static_cast<double*>(grad));
   return hipGetLastError();
 }
 

@@ -266,6 +266,8 @@ struct FitFusedArgs {
   double* rmsd;
   double* U;               // 9 per frame or null
   double* tvec;            // 6 per frame or null
+  const double* gout = nullptr;  // gradient only: d loss / d RMSD per frame
+  void* grad = nullptr;          // [frame][nsel][3], FP64 or FP32
 };
 constexpr int FIT_SINGLE_ATOMS = 128;   // up to here a lane takes single atoms, beyond quads
 constexpr int FIT_MANY_FRAMES = 16384;  // from here a wave takes several small frames
@@ -274,6 +276,9 @@ constexpr int FIT_INREF_FRAMES = 512;   // more frames: the reference is prepare
 bool rmsd_fit_fused_fits(int natom, int nsel, int nframes, int mode);
 bool rmsd_fit_inref_fits(int natom, int nsel, int nframes, int mode);
 hipError_t rmsd_launch_fit_fused(const FitFusedArgs& a, hipStream_t s);
+// The gradient of the fit (mode 0, no selection; rmsd, U, tvec unused) the same way.
+bool rmsd_fit_grad_fits(const FrameSetDev& fs);
+hipError_t rmsd_launch_fit_grad_fused(const FitFusedArgs& a, bool f32, hipStream_t s);
 
 // Fit of target frame f of T to reference frame f of R, every f (k_fit.hip,
 // k_fit_pairs): the 'reftraj' and 'previous' reference modes of
@@ -460,7 +465,7 @@ hipError_t rmsd_launch_ref_prep(const FrameSetDev& fs, int f, const double* rmas
 // Gradients (k_grad.hip).
 hipError_t rmsd_launch_fit_grad(const FrameSetDev& fs, const double* mass, const double* ref,
                                 const double* xform, const double* rmsd, const double* gout,
-                                const double* consts, double* grad, hipStream_t s);
+                                const double* consts, void* grad, bool f32, hipStream_t s);
 hipError_t rmsd_launch_center(const FrameSetDev& fs, const double* w, double* xc, double* g,
                               hipStream_t s);
 hipError_t rmsd_launch_pair_grad(const double* XA, const double* XB, const double* gA,

@@ -348,6 +348,10 @@ int rmsd_symm(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frames* ref, 
  * theorem: w_k (x~_k - U^T y~_k) / (M RMSD_f) per atom; 0 where RMSD_f = 0. */
 int rmsd_fit_backward(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frames* ref,
                       int ref_frame, int use_mass, const double* grad_rmsd, double* grad_xyz);
+/* The same gradient, computed in FP64 and rounded to FP32 as it is stored (for
+ * callers whose coordinates and their gradients are FP32). */
+int rmsd_fit_backward_f32(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frames* ref,
+                          int ref_frame, int use_mass, const double* grad_rmsd, float* grad_xyz);
 
 /* Gradient of a full pairwise block (rows = A as targets, columns = B as
  * references, as in rmsd_pairwise with ref != NULL, fit mode): for

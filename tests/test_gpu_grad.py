@@ -131,3 +131,34 @@ def test_differentiation_workload_sizes(oracle, ctx):
             _, gi = oracle_target_grad(oracle, X[i].astype(np.float64), X[512 + j].astype(np.float64), m, True)
             e += gi
         assert np.abs(ga[i].cpu().numpy() - e).max() <= 1e-9 * np.abs(e).max()
+
+
+@pytest.mark.parametrize("F", [3, 700])
+@pytest.mark.parametrize("n", [2, 5, 64, 65, 128, 129, 259, 513, 1027, 2051, 3075, 8192, 8193])
+def test_fit_backward_in_registers(ctx, n, F):
+    """The one-launch gradient (no selection) against the separate kernels (an
+    identity selection takes them) at the edges of its sizes, FP64, and its FP32
+    form against its FP64 one; a frame equal to the reference has no gradient."""
+    import ctypes as C
+    import torch
+    import cpptraj_amd as ca
+    X = dev(synth.noisy(n, F, n, 1.0)) if n * F < 3000000 else dev(synth.noisy(n, 9, n, 1.0))
+    F = X.shape[0]
+    m = dev(synth.masses(np.random.default_rng(n), n))
+    gr = torch.linspace(-1.0, 2.0, F, dtype=torch.float64, device="cuda")
+    sel = torch.arange(n, dtype=torch.int32, device="cuda")
+    ref = X[1:2].clone()
+    out = {}
+    for key, s, fn, dt in (("new", None, ctx._L.rmsd_fit_backward, torch.float64),
+                           ("f32", None, ctx._L.rmsd_fit_backward_f32, torch.float32),
+                           ("old", sel, ctx._L.rmsd_fit_backward, torch.float64)):
+        d, r = ca.frames_desc(X, s, m), ca.frames_desc(ref, s, m)
+        out[key] = torch.full((F, n, 3), 9.0, dtype=dt, device="cuda")
+        ctx.check(fn(ctx.handle, C.byref(d), C.byref(r), 0, 1, C.c_void_p(gr.data_ptr()),
+                     C.c_void_p(out[key].data_ptr())))
+    new, old = out["new"].cpu().numpy(), out["old"].cpu().numpy()
+    assert torch.equal(out["f32"], out["new"].float())
+    assert np.isfinite(new).all()
+    if n > 2:  # two atoms: the rotation is not unique
+        rest = [f for f in range(F) if f != 1]
+        assert np.abs(new[rest] - old[rest]).max() <= 1e-9 * np.abs(old[rest]).max()
