@@ -1085,13 +1085,30 @@ int rmsd_avgcorr(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frames* re
   for (int i = 0; i < nw; ++i) wmap[ws[i]] = i;
   std::vector<int32_t> cnt((size_t)F + 2, 0);  // cnt[w + 1] = windows <= w
   for (int64_t w = 0; w <= F; ++w) cnt[w + 1] = cnt[w] + (wmap[w] >= 0 ? 1 : 0);
+  auto crossed = [&](int ti, int tj) {
+    const int64_t base = (int64_t)T * (ti - tj);
+    const int64_t lo = std::max<int64_t>(1, base - (T - 1)), hi = std::min<int64_t>(F, base + T - 1);
+    return lo <= hi && cnt[hi + 1] > cnt[lo];
+  };
   std::vector<int2> tiles;
-  for (int ti = 0; ti < ntile; ++ti)
-    for (int tj = 0; tj <= ti; ++tj) {
-      const int64_t base = (int64_t)T * (ti - tj);
-      const int64_t lo = std::max<int64_t>(1, base - (T - 1)), hi = std::min<int64_t>(F, base + T - 1);
-      if (lo <= hi && cnt[hi + 1] > cnt[lo]) tiles.push_back(make_int2(ti, tj));
-    }
+  int ngram = 0;
+  if (first) {
+    for (int ti = 0; ti < ntile; ++ti)
+      for (int tj = 0; tj <= ti; ++tj)
+        if (crossed(ti, tj)) tiles.push_back(make_int2(ti, tj));
+  } else {
+    // The tiles on and next to the diagonal, then the others in bands of
+    // GROUP row tiles, column by column (ac_gram's order).
+    for (int ti = 0; ti < ntile; ++ti)
+      for (int tj = std::max(0, ti - 1); tj <= ti; ++tj)
+        if (crossed(ti, tj)) tiles.push_back(make_int2(ti, tj));
+    const size_t near = tiles.size();
+    for (int b0 = 0; b0 < ntile; b0 += GROUP)
+      for (int tj = 0; tj < std::min(ntile, b0 + GROUP); ++tj)
+        for (int ti = std::max(b0, tj + 2); ti < std::min(ntile, b0 + GROUP); ++ti)
+          if (crossed(ti, tj)) tiles.push_back(make_int2(ti, tj));
+    ngram = (int)(tiles.size() - near);
+  }
   AvgPrefixArgs a;
   a.fs = to_dev(*frames);
   a.mass = use_mass ? frames->mass : nullptr;
@@ -1121,6 +1138,8 @@ int rmsd_avgcorr(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frames* re
   a.wmap = dmap;
   a.tiles = dtiles;
   a.ntiles = (int)tiles.size();
+  a.ngram = ngram;
+  a.gram_per_xcd = (ngram + NXCD - 1) / NXCD;
   a.ntile = ntile;
   a.tile = T;
   a.yref = nullptr;

@@ -237,6 +237,7 @@ constexpr int AC_THREADS = 256;
 constexpr int AC_TILE = 64;    // prefix rows per tile side
 constexpr int AC_KC = 32;      // coordinates per LDS stage
 constexpr int AC_LD = AC_TILE + 1;
+constexpr int AC_XCDS = 8;
 
 __global__ __launch_bounds__(AC_THREADS) void k_ac_chunksum(AvgPrefixArgs a) {
   const int j = blockIdx.x * AC_THREADS + threadIdx.x;
@@ -359,17 +360,68 @@ __global__ __launch_bounds__(64) void k_ac_rows(AvgPrefixArgs a) {
     for (int q = 0; q < 13; ++q) a.rows[i * 13 + q] = r[q];
 }
 
-// One 64 x 64 tile of (i, j) prefix-row pairs.  Thread (ty, tx) = (t / 16,
-// t % 16) owns rows i0 + ty + 16 a and j0 + tx + 16 b (a, b < 4).
-__global__ __launch_bounds__(AC_THREADS) void k_ac_tiles(AvgPrefixArgs a) {
-  // [2][KC][65] staged coordinates (odd row stride: conflict-free transposed
-  // stores), later the RMSDs [64][65].
-  __shared__ double sm[2 * AC_KC * AC_LD];
-  static_assert(2 * AC_KC * AC_LD >= AC_TILE * AC_LD, "RMSD tile does not fit");
+// The fit of one averaged frame from the difference form's pieces: d2 = sum
+// m |P_i - P_j|^2, the row moments ri and rj, the constants row cm and the
+// reference constants K.
+__device__ __forceinline__ double ac_fit(double d2, const double* ri, const double (&rj)[13],
+                                         const double* cm, const double* K, double iW, double w) {
+  const double W = K[4];
+  if (W < RMSD_SMALL) return -1.0;
+  // 1 / w to the last bit or two: the hardware reciprocal, refined twice
+  double iw = __builtin_amdgcn_rcp(w);
+  iw = fma(iw, fma(-w, iw, 1.0), iw);
+  iw = fma(iw, fma(-w, iw, 1.0), iw);
+  double dc[3], c[3];
+#pragma unroll
+  for (int e = 0; e < 3; ++e) {
+    dc[e] = (ri[e] - rj[e]) * (iw * iW);
+    c[e] = dc[e] + cm[e] * iW;
+  }
+  double R[9];
+#pragma unroll
+  for (int e = 0; e < 9; ++e) R[e] = (ri[3 + e] - rj[3 + e]) * iw + cm[3 + e] - c[e / 3] * K[e % 3];
+  const double sx = d2 * (iw * iw) + 2.0 * (ri[12] - rj[12]) * iw + cm[12] -
+                    W * (dc[0] * dc[0] + dc[1] * dc[1] + dc[2] * dc[2]);
+  return rmsd_dev::qcp_rmsd_fast(R, 0.5 * (sx + K[3]), iW, 1);
+}
+
+// Sums of a tile's RMSDs rr[64][AC_LD] along its diagonals: thread dd + 63
+// takes local diagonal dd = il - jl.
+__device__ __forceinline__ void ac_diagonals(const AvgPrefixArgs& a, const double* rr, int ti,
+                                             int tj) {
+  const int64_t i0 = (int64_t)ti * AC_TILE, j0 = (int64_t)tj * AC_TILE;
+  const int64_t nrow = a.fs.nframes + 1;
+  const int t = threadIdx.x;
+  if (t >= 2 * AC_TILE - 1) return;
+  const int dd = t - (AC_TILE - 1);
+  const int64_t w = (i0 - j0) + dd;
+  if (!(w >= 1 && w < nrow && a.wmap[w] >= 0)) return;
+  double s1 = 0.0, s2 = 0.0;
+  const int il0 = dd > 0 ? dd : 0, il1 = dd < 0 ? AC_TILE + dd : AC_TILE;
+  for (int il = il0; il < il1; ++il) {
+    const double r = rr[il * AC_LD + il - dd];
+    s1 += r;
+    s2 += r * r;
+  }
+  // Slot of this tile among the two j tiles that diagonal w crosses in row
+  // tile ti.
+  const int half = tj - (ti - (int)((w + AC_TILE - 1) / AC_TILE));
+  double* o = a.part + (((int64_t)a.wmap[w] * a.ntile + ti) * 2 + half) * 2;
+  o[0] = s1;
+  o[1] = s2;
+}
+
+// One 64 x 64 tile of (i, j) prefix-row pairs, distances from the differences.
+// Thread (ty, tx) = (t / 16, t % 16) owns rows i0 + ty + 16 a and j0 + tx + 16 b
+// (a, b < 4).  For the tiles on and next to the diagonal (ac_gram takes the
+// others).
+// sm: [2][KC][65] staged coordinates (odd row stride: conflict-free transposed
+// stores), later the RMSDs [64][65].
+constexpr int AC_LDS = 2 * AC_KC * AC_LD;
+static_assert(AC_LDS >= AC_TILE * AC_LD, "RMSD tile does not fit");
+__device__ __forceinline__ void ac_direct(const AvgPrefixArgs& a, int ti, int tj, double* sm) {
   double* si = sm;
   double* sj = sm + AC_KC * AC_LD;
-  const int2 tile = a.tiles[blockIdx.x];
-  const int ti = tile.x, tj = tile.y;
   const int64_t i0 = (int64_t)ti * AC_TILE, j0 = (int64_t)tj * AC_TILE;
   const int64_t nrow = a.fs.nframes + 1;
   const int t = threadIdx.x, ty = t >> 4, tx = t & 15;
@@ -409,60 +461,174 @@ __global__ __launch_bounds__(AC_THREADS) void k_ac_tiles(AvgPrefixArgs a) {
     __syncthreads();
   }
   // Fits of the pairs on window diagonals.
-  const double* K = a.consts;  // sum w y (3), sum w |y|^2, W
-  const double W = K[4];
   const double* cm = a.rows + nrow * 13;
+  const double iW = 1.0 / a.consts[4];
   double* rr = sm;
-  for (int p = 0; p < 4; ++p)
-    for (int q = 0; q < 4; ++q) {
-      const int il = ty + 16 * p, jl = tx + 16 * q;
-      const int64_t i = i0 + il, j = j0 + jl;
-      const int64_t w = i - j;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int jl = tx + 16 * q;
+    const int64_t j = j0 + jl;
+    double rj[13];
+#pragma unroll
+    for (int e = 0; e < 13; ++e) rj[e] = a.rows[(j < nrow ? j : 0) * 13 + e];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const int il = ty + 16 * p;
+      const int64_t i = i0 + il, w = i - j;
       double r = 0.0;
-      if (w >= 1 && i < nrow && a.wmap[w] >= 0) {
-        if (W < RMSD_SMALL) {
-          r = -1.0;
-        } else {
-          const double dw = (double)w;
-          const double* ri = a.rows + i * 13;
-          const double* rj = a.rows + j * 13;
-          double dc[3], c[3];
-          for (int e = 0; e < 3; ++e) {
-            dc[e] = (ri[e] - rj[e]) / (dw * W);
-            c[e] = dc[e] + cm[e] / W;
-          }
-          double R[9];
-          for (int e = 0; e < 9; ++e)
-            R[e] = (ri[3 + e] - rj[3 + e]) / dw + cm[3 + e] - c[e / 3] * K[e % 3];
-          const double sx = acc[p][q] / (dw * dw) + 2.0 * (ri[12] - rj[12]) / dw + cm[12] -
-                            W * (dc[0] * dc[0] + dc[1] * dc[1] + dc[2] * dc[2]);
-          const double E0 = 0.5 * (sx + K[3]);
-          r = rmsd_dev::qcp_rmsd(R, E0, W, 1);
-        }
-      }
+      if (w >= 1 && i < nrow && a.wmap[w] >= 0)
+        r = ac_fit(acc[p][q], a.rows + i * 13, rj, cm, a.consts, iW, (double)w);
       rr[il * AC_LD + jl] = r;
     }
+  }
   __syncthreads();
-  // Diagonal sums: thread dd + 63 takes local diagonal dd = il - jl.
-  if (t < 2 * AC_TILE - 1) {
-    const int dd = t - (AC_TILE - 1);
-    const int64_t w = (i0 - j0) + dd;
-    if (w >= 1 && w < nrow && a.wmap[w] >= 0) {
-      double s1 = 0.0, s2 = 0.0;
-      const int il0 = dd > 0 ? dd : 0, il1 = dd < 0 ? AC_TILE + dd : AC_TILE;
-      for (int il = il0; il < il1; ++il) {
-        const double r = rr[il * AC_LD + il - dd];
-        s1 += r;
-        s2 += r * r;
+  ac_diagonals(a, rr, ti, tj);
+}
+
+// A tile two or more tiles off the diagonal (windows of at least 65 frames):
+// the distances as a Gram product on FP64 MFMA, one multiply-add per coordinate
+// and pair instead of a difference and a multiply-add.  Rows are taken about the
+// middle row m of the column tile, q_i = P_i - P_m, p_j = P_j - P_m:
+//   |P_i - P_j|^2 = |q_i|^2 + |p_j|^2 - 2 q_i . p_j.
+// p_j reaches over at most 32 frames and q_i over about w of them, so what the
+// sum cancels is of the size of the distance itself; where a trajectory makes
+// |P_i - P_j| small against |p_j|, the rounding left, eps |p_j|^2 / w^2 with
+// |p_j| <= 32 frames' deviation and w >= 65, is below eps times the sum
+// m |mu - mu_c|^2 that the fit adds to it.  Nearer the diagonal that does not
+// hold, hence ac_direct there.
+//
+// Each of the four waves owns 32 x 32 pairs, four 16 x 16 blocks; a stage of 32
+// coordinates of the 128 rows goes to LDS shifted, the next stage's loads in
+// flight meanwhile.  Bound by the FP64 matrix
+// rate and, after it, the fits' vector FP64.  Tiles come in bands of eight row
+// tiles, an XCD's workgroups in one run of that order, so that tiles running
+// side by side share rows in its L2.  10,000 frames x 300 atoms, all windows: the
+// whole call 2.43 ms against 4.80 with every tile's distances from the
+// differences; MFMA pipes 54 % busy and vector issue 27 % at 2.1 GHz, three waves
+// per SIMD (four spill: 3.36 ms).  The tiles near the diagonal run in the same
+// launch: 314 of 12,400, alone on the chip they took 286 us.
+typedef __attribute__((ext_vector_type(4))) double f64x4;
+
+__device__ __forceinline__ void ac_gram(const AvgPrefixArgs& a, int ti, int tj, double* sm,
+                                        double (*norm)[2 * AC_TILE]) {
+  double* si = sm;
+  double* sj = sm + AC_KC * AC_LD;
+  const int64_t i0 = (int64_t)ti * AC_TILE, j0 = (int64_t)tj * AC_TILE;
+  const int64_t nrow = a.fs.nframes + 1;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int lc = t & (AC_KC - 1), lr = t >> 5;
+  const double* mid = a.P + (j0 + AC_TILE / 2) * a.k;  // tj < ti: a whole tile of rows
+  // Uniform bases and one 32-bit lane offset for all sixteen rows.
+  const double* bi = a.P + i0 * a.k;
+  const double* bj = a.P + j0 * a.k;
+  const int lo = lr * a.k + lc;
+  const int rows = (int)(nrow - i0 < AC_TILE ? nrow - i0 : AC_TILE);
+  const int kfull = rows == AC_TILE ? a.k - AC_KC : -1;  // stages before it need no checks
+  double vi[8], vj[8], vm;
+  auto fetch = [&](int k0) {
+    if (k0 <= kfull) {  // uniform
+      vm = gp(mid + k0)[lc];
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        vi[r] = gp(bi + (int64_t)(8 * r) * a.k + k0)[lo];
+        vj[r] = gp(bj + (int64_t)(8 * r) * a.k + k0)[lo];
       }
-      // Slot of this tile among the two j tiles that diagonal w crosses in
-      // row tile ti.
-      const int half = tj - (ti - (int)((w + AC_TILE - 1) / AC_TILE));
-      double* o = a.part + (((int64_t)a.wmap[w] * a.ntile + ti) * 2 + half) * 2;
-      o[0] = s1;
-      o[1] = s2;
+      return;
+    }
+    const bool in = k0 + lc < a.k;
+    vm = in ? gp(mid + k0)[lc] : 0.0;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      vi[r] = in && lr + 8 * r < rows ? gp(bi + (int64_t)(8 * r) * a.k + k0)[lo] : vm;
+      vj[r] = in ? gp(bj + (int64_t)(8 * r) * a.k + k0)[lo] : vm;
+    }
+  };
+  // The rows' squares: thread t sums half of each stage's coordinates (t / 128)
+  // of row t % 128 of the i rows, then the j rows.
+  const double* srow = (t & 64 ? sj : si) + (t & 63) + (t >> 7) * (AC_KC / 2) * AC_LD;
+  double sq = 0.0;
+  f64x4 acc[2][2];
+#pragma unroll
+  for (int p = 0; p < 2; ++p)
+#pragma unroll
+    for (int q = 0; q < 2; ++q) acc[p][q] = f64x4{0.0, 0.0, 0.0, 0.0};
+  const int ri0 = 32 * (wave >> 1) + (lane & 15), cj0 = 32 * (wave & 1) + (lane & 15);
+  fetch(0);
+  for (int k0 = 0; k0 < a.k; k0 += AC_KC) {
+    __syncthreads();  // the last stage's reads
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      si[lc * AC_LD + lr + 8 * r] = vi[r] - vm;
+      sj[lc * AC_LD + lr + 8 * r] = vj[r] - vm;
+    }
+    __syncthreads();
+    if (k0 + AC_KC < a.k) fetch(k0 + AC_KC);
+#pragma unroll
+    for (int c = 0; c < AC_KC / 2; ++c) sq = fma(srow[c * AC_LD], srow[c * AC_LD], sq);
+#pragma unroll
+    for (int c = 0; c < AC_KC; c += 4) {
+      const int kk = (c + (lane >> 4)) * AC_LD;
+      double av[2], bv[2];
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        av[p] = si[kk + ri0 + 16 * p];
+        bv[p] = sj[kk + cj0 + 16 * p];
+      }
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+          acc[p][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[p], bv[q], acc[p][q], 0, 0, 0);
     }
   }
+  norm[t >> 7][t & 127] = sq;
+  __syncthreads();  // and the last stage's reads: sm becomes the RMSD tile
+  const double* cm = a.rows + nrow * 13;
+  const double iW = 1.0 / a.consts[4];
+  // The accumulators hold row lane / 16 + 4 v, column lane % 16, in item v.
+#pragma unroll 1
+  for (int q = 0; q < 2; ++q) {
+    const int jl = cj0 + 16 * q;
+    const int64_t j = j0 + jl;
+    double rj[13];
+#pragma unroll
+    for (int e = 0; e < 13; ++e) rj[e] = gp(a.rows)[j * 13 + e];
+    const double nj = norm[0][AC_TILE + jl] + norm[1][AC_TILE + jl];
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int il = 32 * (wave >> 1) + 16 * p + (lane >> 4) + 4 * v;
+        const int64_t i = i0 + il, w = i - j;
+        double r = 0.0;
+        if (i < nrow && a.wmap[w] >= 0) {
+          const double g = q == 0 ? acc[p][0][v] : acc[p][1][v];
+          const double d2 = fmax(norm[0][il] + norm[1][il] + nj - 2.0 * g, 0.0);
+          r = ac_fit(d2, a.rows + i * 13, rj, cm, a.consts, iW, (double)w);
+        }
+        sm[il * AC_LD + jl] = r;
+      }
+  }
+  __syncthreads();
+  ac_diagonals(a, sm, ti, tj);
+}
+
+// The tiles near the diagonal first: they take longest.
+__global__ __launch_bounds__(AC_THREADS) __attribute__((amdgpu_waves_per_eu(3))) void k_ac_tiles(
+    AvgPrefixArgs a) {
+  __shared__ double sm[AC_LDS];
+  __shared__ double norm[2][2 * AC_TILE];
+  const int near = a.ntiles - a.ngram;
+  if ((int)blockIdx.x < near) {
+    const int2 tile = a.tiles[blockIdx.x];
+    ac_direct(a, tile.x, tile.y, sm);
+    return;
+  }
+  const int b = (int)blockIdx.x - near;
+  const int w = (b % AC_XCDS) * a.gram_per_xcd + b / AC_XCDS;
+  if (w >= a.ngram) return;  // the whole workgroup
+  const int2 tile = a.tiles[near + w];
+  ac_gram(a, tile.x, tile.y, sm, norm);
 }
 
 // Mean and standard deviation per window from the per-tile sums, in a fixed
@@ -725,7 +891,9 @@ hipError_t rmsd_launch_avgcorr_tiles(const AvgPrefixArgs& a, hipStream_t s) {
     hipLaunchKernelGGL(k_ac_firstref, dim3(a.nwin), dim3(64), 0, s, a);
     hipLaunchKernelGGL(k_ac_tiles_first, dim3(a.ntiles), dim3(AC_THREADS), 0, s, a);
   } else {
-    hipLaunchKernelGGL(k_ac_tiles, dim3(a.ntiles), dim3(AC_THREADS), 0, s, a);
+    if (a.ngram > a.ntiles || a.gram_per_xcd * AC_XCDS < a.ngram) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_ac_tiles, dim3(a.ntiles - a.ngram + a.gram_per_xcd * AC_XCDS),
+                       dim3(AC_THREADS), 0, s, a);
   }
   return hipGetLastError();
 }

@@ -381,6 +381,8 @@ struct AvgPrefixArgs {
   const int* wmap;        // [F+1] window index of a window size, else -1
   const int2* tiles;      // (row tile, column tile) pairs to run
   int ntiles;
+  int ngram = 0;          // fixed reference: the last ngram tiles are two or more
+  int gram_per_xcd = 0;   // tiles off the diagonal (tile.x - tile.y >= 2); ngram / XCDs, up
   int ntile;              // row tiles: ceil((F+1) / 64)
   double* part;           // [nwin][ntile][2][2] per-tile sums of RMSD and RMSD^2
   int tile;               // frames per tile side (64 fixed reference, 32 'first')

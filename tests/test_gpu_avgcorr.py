@@ -192,3 +192,31 @@ def test_avgcorr_errors(ctx):
         _avgcorr(ca, ctx, Z, ref_frames=Z[:1], method="running")
     with pytest.raises(ca.RmsdError, match="unknown rmsavgcorr method"):
         ctx.check(ctx._L.rmsd_avgcorr_set_method(ctx.handle, 7))
+
+
+@pytest.mark.parametrize("F", [126, 127, 128, 190, 191, 192, 256, 321])
+@pytest.mark.parametrize("n,use_mass,offset", [(5, False, 1), (11, True, 1), (32, False, 70), (43, True, 2)])
+def test_avgcorr_gram_tile_edges(ctx, F, n, use_mass, offset):
+    """Tiles off the diagonal (distances as a product): frame counts at the
+    edges of the 64-row tiles, coordinates that leave a stage of 32 unfilled and
+    windows that cross only some tiles, against the running sum.  A drift of 8 A
+    over the trajectory makes the prefix sums large against their differences."""
+    import torch
+
+    import cpptraj_amd as ca
+    rng = np.random.default_rng(F + n)
+    X3 = synth.noisy(F + n, 1, n, 0.0) + rng.normal(scale=0.5, size=(F, n, 3)) + np.linspace(0, 8, F)[:, None, None]
+    X = torch.as_tensor(X3.reshape(F, -1).astype(np.float32)).cuda()
+    R = X[3:4].clone()
+    m = torch.as_tensor(synth.masses(rng, n)).cuda()
+    kw = dict(ref_frames=R, mass=m, use_mass=use_mass, offset=offset)
+    w, ct, sd = _avgcorr(ca, ctx, X, method="prefix", **kw)
+    w2, ct2, sd2 = _avgcorr(ca, ctx, X, method="running", **kw)
+    assert np.array_equal(w, w2)
+    # The windows those tiles hold: 65 frames and more (window 1 also has the
+    # reference fitted to itself, noise of sqrt(eps E0 / M) on either side).
+    far = torch.as_tensor(w >= 65).cuda()
+    assert float((ct - ct2)[far].abs().max()) <= TOL
+    # SD = sqrt(mean(r^2) - mean(r)^2): rounding of the two means, ~1e-15 r^2,
+    # under the root.
+    assert float((sd ** 2 - sd2 ** 2)[far].abs().max()) <= 1e-12 * float(ct2.max()) ** 2
