@@ -322,7 +322,7 @@ struct Packed {
 };
 
 int prepare_set(rmsd_ctx* c, const FrameSetDev& fs, const double* cmass, const double* smass,
-                int prec, int Kp, const double* T, const double* gT, const double* M,
+                int prec, int Kp, const double* T, const double* gT, double* M, bool sum_weights,
                 const char* tag, Packed* out) {
   const int CH = chunk_atoms(prec);
   // Padded to whole row and column tiles: 64 and rmsd_pairwise_tile_cols.
@@ -361,6 +361,7 @@ int prepare_set(rmsd_ctx* c, const FrameSetDev& fs, const double* cmass, const d
   a.cen = out->cen;
   a.total_mass = M;
   if (prec != PREC_F64) a.bound = rmsd_bound_coef(prec, a.KB);
+  if (sum_weights) a.wsum = M;
   HIP_TRY(c, rmsd_launch_prep(a, c->stream));
   return RMSD_OK;
 }
@@ -410,18 +411,18 @@ int pairwise_impl(rmsd_ctx* c, const FrameSetDev& A, const FrameSetDev& B, int t
     T = (double*)scratch(c, "pair.template", sizeof(double) * 3 * Kp, &st);
     if (!T) return st;
   }
-  SetupArgs s{};
-  s.fs = B;  // template: first column (reference) frame
-  s.f0 = 0;
-  s.cmass = bmass;
-  s.smass = wmass;
-  s.Kp = Kp;
-  s.T = T;
-  s.P = P;
-  s.gT = gT;
-  s.total_mass = M;
-  HIP_TRY(c, rmsd_launch_setup(s, c->stream));
   if (mixed) {
+    SetupArgs s{};
+    s.fs = B;  // template: first column (reference) frame
+    s.f0 = 0;
+    s.cmass = bmass;
+    s.smass = wmass;
+    s.Kp = Kp;
+    s.T = T;
+    s.P = P;
+    s.gT = gT;
+    s.total_mass = M;
+    HIP_TRY(c, rmsd_launch_setup(s, c->stream));
     // Mean structure of evenly spaced reference frames as the template.
     const int nsamp = std::min(TEMPLATE_SAMPLES, B.nframes);
     double* part = (double*)scratch(c, "pair.tmplpart", sizeof(double) * 3 * Kp * nsamp, &st);
@@ -430,10 +431,11 @@ int pairwise_impl(rmsd_ctx* c, const FrameSetDev& A, const FrameSetDev& B, int t
   }
 
   Packed pa, pb;
-  if ((st = prepare_set(c, A, amass, wmass, prec, Kp, T, gT, M, "A", &pa)) != RMSD_OK) return st;
+  if ((st = prepare_set(c, A, amass, wmass, prec, Kp, T, gT, M, !mixed, "A", &pa)) != RMSD_OK)
+    return st;
   if (tri) {
     pb = pa;
-  } else if ((st = prepare_set(c, B, bmass, wmass, prec, Kp, T, gT, M, "B", &pb)) != RMSD_OK) {
+  } else if ((st = prepare_set(c, B, bmass, wmass, prec, Kp, T, gT, M, false, "B", &pb)) != RMSD_OK) {
     return st;
   }
   PairArgs p;

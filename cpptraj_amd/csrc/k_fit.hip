@@ -53,41 +53,13 @@ __device__ __forceinline__ float fcoord(const FrameSetDev& fs, int64_t f, int k,
 constexpr int REF_THREADS = 1024;
 constexpr int REF_STAGE = 2048;  // masses per LDS stage
 
-__device__ __forceinline__ void mass_chain(const double* m, int n, int ldr, double* wpad,
-                                           double* stage, double* W) {
-  double s = 0.0;
-  for (int k0 = 0; k0 < ldr; k0 += REF_STAGE) {
-    const int c = ldr - k0 < REF_STAGE ? ldr - k0 : REF_STAGE;
-    for (int k = threadIdx.x; k < c; k += blockDim.x) {
-      const double v = k0 + k < n ? m[k0 + k] : 0.0;
-      stage[k] = v;
-      if (wpad) wpad[k0 + k] = v;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      const int real = n - k0 < c ? n - k0 : c;  // the padding is not added
-      int k = 0;
-      for (; k + 16 <= real; k += 16) {
-        double v[16];
-#pragma unroll
-        for (int e = 0; e < 16; ++e) v[e] = stage[k + e];
-#pragma unroll
-        for (int e = 0; e < 16; ++e) s += v[e];
-      }
-      for (; k < real; ++k) s += stage[k];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) *W = s;
-}
-
 __global__ __launch_bounds__(REF_THREADS) void k_ref_prep(FrameSetDev fs, int f, const double* rmass,
                                                           const double* tmass, int center, int ldr,
                                                           double* ref_out, double* ref_trans,
                                                           double* consts, double* wpad) {
   __shared__ double sm[REF_STAGE];
   if (blockIdx.x == 1) {
-    mass_chain(tmass, fs.nsel, ldr, wpad, sm, consts + 4);
+    rmsd_dev::mass_chain<REF_STAGE>(tmass, fs.nsel, ldr, wpad, sm, consts + 4);
     return;
   }
   double* red = sm;  // 4 sums per wave

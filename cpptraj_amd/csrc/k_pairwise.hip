@@ -31,6 +31,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <type_traits>
+// Contracted by expression: every kernel here gives a pair the same bits,
+// whatever tile shape it sits in (batched and single calls agree).
+#pragma clang fp contract(on)
 #include "rmsd_device.hpp"
 #include "rmsd_kernels.hpp"
 
@@ -279,6 +282,50 @@ __device__ __forceinline__ void pair_epilogue(const PairArgs& args,
   }
 }
 
+// The FP64 epilogue of one 16 x 16 block: pair_epilogue's solves, to the same
+// bits, with the Newton steps of a lane's four pairs side by side (each pair
+// stops where it would alone): a block of a small matrix has its SIMD to itself
+// and waits for every dependent step otherwise.
+__device__ __forceinline__ void block_epilogue_f64(const PairArgs& args, f64x4 (&acc)[3][3],
+                                                   int64_t fbA, int64_t fbB, int lane) {
+  const auto gA = gp(args.gA);
+  const double M = gp(args.total_mass)[0];
+  const int64_t j = fbB * 16 + (lane & 15);
+  const double gj = j < args.FB ? gp(args.gB)[j] : 0.0;
+  bool ok[4], go[4];
+  double E0[4], lam[4];
+  rmsd_dev::QcpCoef co[4];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const int64_t i = fbA * 16 + (lane >> 4) + 4 * v;
+    ok[v] = go[v] = j < args.FB && i < args.FA && (!args.tri || i < j);
+    E0[v] = lam[v] = 0.5 * ((i < args.FA ? gA[i] : 0.0) + gj);
+    double R[9];  // rows are the reference in the triangle layout
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+      for (int d = 0; d < 3; ++d) R[3 * c + d] = args.tri ? acc[d][c][v] : acc[c][d][v];
+    co[v] = rmsd_dev::qcp_coefficients(R);
+  }
+  for (int it = 0; it < 50 && (go[0] || go[1] || go[2] || go[3]); ++it) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const double next = rmsd_dev::qcp_step(co[v], lam[v]);
+      const bool done = fabs(next - lam[v]) < fabs(1e-11 * next);
+      lam[v] = go[v] ? next : lam[v];
+      go[v] = go[v] && !done;
+    }
+  }
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    if (!ok[v]) continue;
+    const int64_t i = fbA * 16 + (lane >> 4) + 4 * v;
+    const int64_t idx = args.tri ? rmsd_dev::tri_index(args.FA, i, j) : i * args.FB + j;
+    gp(args.out)[idx] =
+        M < RMSD_SMALL ? -1.0f : (float)rmsd_dev::rmsd_from_lambda(E0[v], lam[v], M, args.clamp);
+  }
+}
+
 // ---- FP64 recomputation of flagged pairs -------------------------------------------
 // The contraction lists every wave with a pair over the tolerance (wlist,
 // nflag[0] entries) and leaves that wave's lane masks.  Here one wave
@@ -458,21 +505,16 @@ __global__ __launch_bounds__(FALLBACK_THREADS, 2) void k_pair_fallback_batch(
   }
 }
 
-// One 64 x 64 tile of frame pairs: contraction over all atom chunks, then
-// the FP64 epilogue.  Shared by the single-matrix and the batched kernels.
-template <int PREC, int WR, int WC, int NWR, int NWC>
-__device__ __forceinline__ void pair_tile(const PairArgs& args, int2 tile, int tile_id) {
+// One wave's (16 WR) x (16 WC) frame pairs (first row block fbA, column block
+// fbB): contraction over all atom chunks, then the FP64 epilogue.  Shared by
+// the single-matrix and the batched kernels.
+template <int PREC, int WR, int WC>
+__device__ __forceinline__ void pair_block(const PairArgs& args, int64_t fbA, int64_t fbB,
+                                           int tile_id, int wave, int nwaves) {
   typedef PrecTraits<PREC> T;
   typedef typename T::acc_t acc_t;
   constexpr int PARTS = T::PARTS;
-  constexpr int TILE_R = 16 * WR * NWR;
-  constexpr int TILE_C = 16 * WC * NWC;
-  const int wave = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
-  const int wr = wave / NWC, wc = wave % NWC;
-  const int64_t fbA = (int64_t)tile.x * (TILE_R / 16) + wr * WR;  // first 16-frame row block
-  const int64_t fbB = (int64_t)tile.y * (TILE_C / 16) + wc * WC;  // first 16-frame col block
-
   const u32x4* A = reinterpret_cast<const u32x4*>(args.A);
   const u32x4* B = reinterpret_cast<const u32x4*>(args.B);
   const int KB = args.KB;
@@ -532,7 +574,18 @@ __device__ __forceinline__ void pair_tile(const PairArgs& args, int2 tile, int t
           for (int d = 0; d < 3; ++d) mma<PREC>(acc[r][q][c][d], ca[r][c], cb[q][d]);
   }
 
-  pair_epilogue<PREC, WR, WC>(args, acc, fbA, fbB, lane, tile_id, wave, NWR * NWC, bl);
+  if constexpr (PREC == PREC_F64 && WR == 1 && WC == 1)
+    block_epilogue_f64(args, acc[0][0], fbA, fbB, lane);
+  else
+    pair_epilogue<PREC, WR, WC>(args, acc, fbA, fbB, lane, tile_id, wave, nwaves, bl);
+}
+
+// A workgroup's tile of NWR x NWC such waves.
+template <int PREC, int WR, int WC, int NWR, int NWC>
+__device__ __forceinline__ void pair_tile(const PairArgs& args, int2 tile, int tile_id) {
+  const int wave = threadIdx.x >> 6;
+  pair_block<PREC, WR, WC>(args, (int64_t)tile.x * (WR * NWR) + wave / NWC * WR,
+                           (int64_t)tile.y * (WC * NWC) + wave % NWC * WC, tile_id, wave, NWR * NWC);
 }
 
 // ---- Operands shared through LDS ---------------------------------------------------
@@ -667,6 +720,28 @@ __global__ __launch_bounds__(64 * NWR * NWC) void k_pairwise(PairArgs args) {
   pair_tile<PREC, WR, WC, NWR, NWC>(args, args.tiles[t], t);
 }
 
+// FP64, single matrix: a workgroup of one wave takes a 16 x 16 block of the
+// pairs of a 64 x 64 tile of the list.  Blocks this small fill the chip from a
+// few hundred frames on (64 x 64 workgroups left 192 of 256 CUs idle at 512 x
+// 512 pairs, and CUs idle in the last round of a few), skip the empty half of
+// the diagonal's tiles, and run three to a SIMD (<= 168 registers), so that one
+// wave's FP64 solves run beside the others' MFMAs.  Bound by FP64 MFMA: 3,001 x
+// 305 429 us (58 TFLOP/s with the preparation) against 489 in eight-wave 64 x 64
+// workgroups of 16 x 32 blocks, 512 frames x 2,000 185 / 586, 101 x 66 14.2 /
+// 35.6, 1,000 x 2,000 457 / 593, 8,000 x 1,200 10.4 / 10.6 ms.  Left to choose
+// its registers the compiler takes 200, two waves per SIMD: 566 us at 3,001 x 305.
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_pairwise_f64(
+    PairArgs args) {
+  const int i = blockIdx.x / args.nxcd;
+  const int t = (blockIdx.x % args.nxcd) * args.per_xcd + i / 16;
+  if (t >= args.ntiles) return;
+  const int2 tile = args.tiles[t];
+  const int64_t fbA = (int64_t)tile.x * 4 + i % 16 / 4, fbB = (int64_t)tile.y * 4 + i % 4;
+  if (fbA * 16 >= args.FA || fbB * 16 >= args.FB) return;
+  if (args.tri && fbA > fbB) return;  // no pair above the diagonal
+  pair_block<PREC_F64, 1, 1>(args, fbA, fbB, t, 0, 1);
+}
+
 // ---- batched matrices ---------------------------------------------------------------
 // Tiles of many independent matrices (one PairArgs per set) in nq queues, one
 // per XCD, each a contiguous, cost-balanced run of the cost-sorted tile list.
@@ -752,8 +827,8 @@ __global__ void k_fill_int(int* p, int n, int v) {
 
 // ---------------------------------------------------------------------------
 // Launchers.  Tile shapes: FP64 waves own 16x32 pairs (72 FP64 accumulators),
-// FP32 and split-BF16 waves 32x48 pairs (216 FP32 accumulators); a workgroup
-// covers 64 x 64 (FP64) or 64 x 96 frame pairs.
+// (16x16 in the single-matrix kernel), FP32 and split-BF16 waves 32x48 pairs (216
+// FP32 accumulators); a workgroup covers 64 x 64 (FP64) or 64 x 96 frame pairs.
 template <int PREC, int WR, int WC, int NWR, int NWC>
 static hipError_t launch_tiles(const PairArgs& a, hipStream_t s) {
   const int nblocks = a.per_xcd * a.nxcd;
@@ -788,9 +863,16 @@ static hipError_t launch_shared(const PairArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
+static hipError_t launch_f64(const PairArgs& a, hipStream_t s) {
+  const int64_t grid = (int64_t)a.per_xcd * a.nxcd * 16;
+  if (grid > 0x7fffffff) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_pairwise_f64, dim3((unsigned)grid), dim3(64), 0, s, a);
+  return hipGetLastError();
+}
+
 hipError_t rmsd_launch_pairwise(int prec, const PairArgs& a, hipStream_t s) {
   switch (prec) {
-    case PREC_F64: return launch_tiles<PREC_F64, 1, 2, 4, 2>(a, s);
+    case PREC_F64: return launch_f64(a, s);
     case PREC_F32: return launch_tiles<PREC_F32, 2, 3, 2, 2>(a, s);
     case PREC_BF16X3: return launch_shared<PREC_BF16X3>(a, s);
     default: return hipErrorInvalidValue;

@@ -111,29 +111,16 @@ __device__ __forceinline__ void template_quad(const double* T, int Kp, int q, do
 }
 
 // ---- template / total weight -----------------------------------------------
+// The total weight, by a workgroup of its own beside the template's (part 1 of
+// two): its chain of additions took 35 us in front of it for 2,000 weights.
+constexpr int WSUM_STAGE = 512;
+__device__ __forceinline__ void setup_weight(const SetupArgs& a) {
+  __shared__ double stage[WSUM_STAGE];
+  rmsd_dev::mass_chain<WSUM_STAGE>(a.smass, a.fs.nsel, a.fs.nsel, nullptr, stage, a.total_mass);
+}
+
 __device__ __forceinline__ void setup_body(const SetupArgs& a) {
   __shared__ double red[16 * (PREP_THREADS / 64)];
-  if (threadIdx.x == 0) {
-    // Sequential running total, rounded as the reference's per-pair sum; the
-    // weights are loaded 16 at a time so that their loads overlap.
-    double tw = 0.0;
-    if (a.smass) {
-      const auto m = gp(a.smass);
-      const int n = a.fs.nsel;
-      int k = 0;
-      for (; k + 16 <= n; k += 16) {
-        double v[16];
-#pragma unroll
-        for (int e = 0; e < 16; ++e) v[e] = m[k + e];
-#pragma unroll
-        for (int e = 0; e < 16; ++e) tw += v[e];
-      }
-      for (; k < n; ++k) tw += m[k];
-    } else {
-      tw = (double)a.fs.nsel;
-    }
-    a.total_mass[0] = tw;
-  }
   if (!a.T) return;
   double cen[3];
   centroid(a.fs, a.f0, a.cmass, red, cen);
@@ -157,7 +144,10 @@ __device__ __forceinline__ void setup_body(const SetupArgs& a) {
   }
 }
 
-__global__ __launch_bounds__(PREP_THREADS) void k_setup(SetupArgs a) { setup_body(a); }
+__global__ __launch_bounds__(PREP_THREADS) void k_setup(SetupArgs a) {
+  if (blockIdx.x == 0) setup_weight(a);
+  else setup_body(a);
+}
 
 // ---- mean-structure template ---------------------------------------------------
 // The MFMA-reduced forms contract deviations D = U x~ - T, and their error
@@ -265,10 +255,11 @@ __global__ __launch_bounds__(PREP_THREADS) void k_tmpl_consts_batch(const SetupA
   tmpl_consts_body(a);
 }
 
-// One workgroup per set (batched matrices).
+// Two workgroups per set (batched matrices).
 __global__ __launch_bounds__(PREP_THREADS) void k_setup_batch(const SetupArgs* sets) {
-  const SetupArgs a = sets[blockIdx.x];
-  setup_body(a);
+  const SetupArgs a = sets[blockIdx.x >> 1];
+  if ((blockIdx.x & 1) == 0) setup_weight(a);
+  else setup_body(a);
 }
 
 // ---- per-frame preparation -----------------------------------------------------
@@ -550,6 +541,16 @@ int64_t prep_grid(int64_t n) {
 
 template <int PREC>
 __global__ __launch_bounds__(PREP_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void k_prep(PrepArgs a) {
+  if (PREC == PREC_F64 && a.wsum && blockIdx.x == gridDim.x - 1) {
+    // FP64 needs no template and the total weight only behind the contraction:
+    // one more workgroup here instead of a launch before.
+    SetupArgs w;
+    w.fs = a.fs;
+    w.smass = a.smass;
+    w.total_mass = a.wsum;
+    setup_weight(w);
+    return;
+  }
   const int64_t f = prep_frame(blockIdx.x);
   if (f < a.Fp) prep_body<PREC>(a, f);
 }
@@ -578,7 +579,7 @@ __global__ __launch_bounds__(PREP_THREADS) __attribute__((amdgpu_waves_per_eu(4)
 }  // namespace
 
 hipError_t rmsd_launch_setup(const SetupArgs& a, hipStream_t s) {
-  hipLaunchKernelGGL(k_setup, dim3(1), dim3(PREP_THREADS), 0, s, a);
+  hipLaunchKernelGGL(k_setup, dim3(a.T ? 2 : 1), dim3(PREP_THREADS), 0, s, a);
   return hipGetLastError();
 }
 
@@ -604,7 +605,7 @@ hipError_t rmsd_launch_template_mean_batch(const SetupArgs* sets, const int* sba
 
 hipError_t rmsd_launch_setup_batch(const SetupArgs* sets, int nsets, hipStream_t s) {
   if (nsets <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_setup_batch, dim3(nsets), dim3(PREP_THREADS), 0, s, sets);
+  hipLaunchKernelGGL(k_setup_batch, dim3(2 * nsets), dim3(PREP_THREADS), 0, s, sets);
   return hipGetLastError();
 }
 
@@ -643,7 +644,8 @@ hipError_t rmsd_launch_prep_batch(int prec, const PrepArgs* sets, const int* fba
 hipError_t rmsd_launch_prep(const PrepArgs& a, hipStream_t s) {
   switch (a.prec) {
     case PREC_F64:
-      hipLaunchKernelGGL(k_prep<PREC_F64>, dim3(prep_grid(a.Fp)), dim3(PREP_THREADS), 0, s, a);
+      hipLaunchKernelGGL(k_prep<PREC_F64>, dim3(prep_grid(a.Fp) + (a.wsum ? 1 : 0)),
+                         dim3(PREP_THREADS), 0, s, a);
       break;
     case PREC_F32:
       hipLaunchKernelGGL(k_prep<PREC_F32>, dim3(prep_grid(a.Fp)), dim3(PREP_THREADS), 0, s, a);

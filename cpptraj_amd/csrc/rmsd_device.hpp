@@ -92,15 +92,20 @@ __device__ __forceinline__ double fast_quot(double n, double d) {
   return n * r;
 }
 
+// One Newton step from lam.
+__device__ __forceinline__ double qcp_step(const QcpCoef& k, double lam) {
+  const double l2 = lam * lam;
+  const double b = (l2 + k.c2) * lam;
+  const double a = b + k.c1;
+  return lam - fast_quot(a * lam + k.c0, 2.0 * l2 * lam + b + a);
+}
+
 // Newton iteration for the largest root, started at E0.
 __device__ __forceinline__ double qcp_lambda(const QcpCoef& k, double E0) {
   double lam = E0;
   for (int it = 0; it < 50; ++it) {
     const double prev = lam;
-    const double l2 = lam * lam;
-    const double b = (l2 + k.c2) * lam;
-    const double a = b + k.c1;
-    lam -= fast_quot(a * lam + k.c0, 2.0 * l2 * lam + b + a);
+    lam = qcp_step(k, prev);
     if (fabs(lam - prev) < fabs(1e-11 * lam)) break;
   }
   return lam;
@@ -351,6 +356,40 @@ __device__ __forceinline__ void block_sum(double (&v)[NV], double* red) {
     v[i] = s;
   }
   __syncthreads();
+}
+
+// *W = the n weights m added one after another, rounded as the reference's
+// running total (n when m is null), by the calling workgroup: a chain of
+// dependent additions, so all its threads stage the weights in LDS (stage: STAGE
+// doubles) and one adds them from there.  wpad (may be null): the weights
+// padded with zeros to `padded` >= n.
+template <int STAGE>
+__device__ __forceinline__ void mass_chain(const double* m, int n, int padded, double* wpad,
+                                           double* stage, double* W) {
+  double s = 0.0;
+  for (int k0 = 0; m && k0 < padded; k0 += STAGE) {
+    const int c = padded - k0 < STAGE ? padded - k0 : STAGE;
+    for (int k = threadIdx.x; k < c; k += blockDim.x) {
+      const double v = k0 + k < n ? m[k0 + k] : 0.0;
+      stage[k] = v;
+      if (wpad) wpad[k0 + k] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      const int real = n - k0 < c ? n - k0 : c;  // the padding is not added
+      int k = 0;
+      for (; k + 16 <= real; k += 16) {
+        double v[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) v[e] = stage[k + e];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) s += v[e];
+      }
+      for (; k < real; ++k) s += stage[k];
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) *W = m ? s : (double)n;
 }
 
 // Packed upper-triangle index without the diagonal (Matrix<T>::calcTriIndex,

@@ -133,6 +133,7 @@ struct PrepArgs {
   double* nrm = nullptr;
   double* cen = nullptr;
   const double* total_mass = nullptr;
+  double* wsum = nullptr;  // FP64: sum of smass (nsel when null) written here, may be null
   BoundCoef bound{};
 };
 
