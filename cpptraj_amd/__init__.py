@@ -134,6 +134,9 @@ def _optional(L):
     if hasattr(L, "rmsd_pairwise_backward"):
         L.rmsd_pairwise_backward.argtypes = [P, FP, FP, C.c_int, P, P, P]
         L.rmsd_pairwise_backward.restype = C.c_int
+    if hasattr(L, "rmsd_pairwise_backward_f32"):
+        L.rmsd_pairwise_backward_f32.argtypes = [P, FP, FP, C.c_int, P, P, P]
+        L.rmsd_pairwise_backward_f32.restype = C.c_int
     if hasattr(L, "rmsd_avgcorr"):
         L.rmsd_avgcorr_windows.argtypes = [C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int32),
                                            C.c_int]

@@ -48,17 +48,23 @@ def _fit_backward(frames, ref, grad_rmsd, mass, use_mass, dtype, ctx=None):
 
 def pairwise_backward(A, B, grad_out, mass=None, use_mass=False, ctx: Context | None = None):
     """FP64 gradients of sum_ij G_ij RMSD(A_i, B_j) with respect to A and B."""
+    return _pairwise_backward(A, B, grad_out, mass, use_mass, torch.float64, ctx)
+
+
+def _pairwise_backward(A, B, grad_out, mass, use_mass, dtype, ctx=None):
+    """pairwise_backward, computed in FP64, grad_out and gradients as `dtype`
+    (float64 or float32)."""
     ctx = ctx or _ctx(A.device)
     L = load_library()
     Ac, Bc = A.contiguous(), B.contiguous()
     da = frames_desc(Ac, None, mass)
     db = frames_desc(Bc, None, mass)
-    ga = torch.empty((A.shape[0], A.shape[1], 3), dtype=torch.float64, device=A.device)
-    gb = torch.empty((B.shape[0], B.shape[1], 3), dtype=torch.float64, device=B.device)
-    G = grad_out.to(torch.float64).contiguous()
-    ctx.check(L.rmsd_pairwise_backward(ctx.handle, C.byref(da), C.byref(db), int(use_mass),
-                                       C.c_void_p(G.data_ptr()), C.c_void_p(ga.data_ptr()),
-                                       C.c_void_p(gb.data_ptr())))
+    ga = torch.empty((A.shape[0], A.shape[1], 3), dtype=dtype, device=A.device)
+    gb = torch.empty((B.shape[0], B.shape[1], 3), dtype=dtype, device=B.device)
+    G = grad_out.to(dtype).contiguous()
+    fn = L.rmsd_pairwise_backward if dtype == torch.float64 else L.rmsd_pairwise_backward_f32
+    ctx.check(fn(ctx.handle, C.byref(da), C.byref(db), int(use_mass), C.c_void_p(G.data_ptr()),
+                 C.c_void_p(ga.data_ptr()), C.c_void_p(gb.data_ptr())))
     return ga, gb
 
 
@@ -109,5 +115,5 @@ class PairwiseRmsd(torch.autograd.Function):
     @staticmethod
     def backward(fctx, G):
         A, B = fctx.saved_tensors
-        ga, gb = pairwise_backward(A, B, G, fctx.mass, fctx.use_mass)
-        return ga.to(A.dtype), gb.to(B.dtype), None, None
+        ga, gb = _pairwise_backward(A, B, G, fctx.mass, fctx.use_mass, A.dtype)
+        return ga, gb, None, None

@@ -101,22 +101,8 @@ int fit_backward(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frames* re
   return RMSD_OK;
 }
 
-}  // namespace
-
-extern "C" {
-
-int rmsd_fit_backward(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frames* ref,
-                      int ref_frame, int use_mass, const double* grad_rmsd, double* grad_xyz) {
-  return fit_backward(ctx, frames, ref, ref_frame, use_mass, grad_rmsd, grad_xyz, false);
-}
-
-int rmsd_fit_backward_f32(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frames* ref,
-                          int ref_frame, int use_mass, const double* grad_rmsd, float* grad_xyz) {
-  return fit_backward(ctx, frames, ref, ref_frame, use_mass, grad_rmsd, grad_xyz, true);
-}
-
-int rmsd_pairwise_backward(rmsd_ctx* ctx, const rmsd_frames* A, const rmsd_frames* B,
-                           int use_mass, const double* grad_out, double* grad_a, double* grad_b) {
+int pairwise_backward(rmsd_ctx* ctx, const rmsd_frames* A, const rmsd_frames* B, int use_mass,
+                      const void* grad_out, void* grad_a, void* grad_b, bool f32) {
   if (!ctx) return RMSD_ERR_ARG;
   int st;
   if ((st = check_frames(ctx, A, "A")) != RMSD_OK) return st;
@@ -141,16 +127,34 @@ int rmsd_pairwise_backward(rmsd_ctx* ctx, const rmsd_frames* A, const rmsd_frame
   if (!cw) return st;
   double* consts = (double*)scratch(ctx, "pair.consts", sizeof(double) * 16, &st);
   if (!consts) return st;
-  SetupArgs s{};
-  s.fs = to_dev(*A);
-  s.smass = w;
-  s.total_mass = consts;
-  HIP_TRY(ctx, rmsd_launch_setup(s, ctx->stream));
-  HIP_TRY(ctx, rmsd_launch_center(to_dev(*A), w, XA, gA, ctx->stream));
-  HIP_TRY(ctx, rmsd_launch_center(to_dev(*B), w, XB, gB, ctx->stream));
+  HIP_TRY(ctx, rmsd_launch_center(to_dev(*A), to_dev(*B), w, XA, XB, gA, gB, consts, ctx->stream));
   HIP_TRY(ctx, rmsd_launch_pair_grad(XA, XB, gA, gB, w, n, FA, FB, consts, grad_out, cw, grad_a,
-                                     grad_b, ctx->stream));
+                                     grad_b, f32, ctx->stream));
   return RMSD_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int rmsd_fit_backward(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frames* ref,
+                      int ref_frame, int use_mass, const double* grad_rmsd, double* grad_xyz) {
+  return fit_backward(ctx, frames, ref, ref_frame, use_mass, grad_rmsd, grad_xyz, false);
+}
+
+int rmsd_fit_backward_f32(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frames* ref,
+                          int ref_frame, int use_mass, const double* grad_rmsd, float* grad_xyz) {
+  return fit_backward(ctx, frames, ref, ref_frame, use_mass, grad_rmsd, grad_xyz, true);
+}
+
+int rmsd_pairwise_backward(rmsd_ctx* ctx, const rmsd_frames* A, const rmsd_frames* B,
+                           int use_mass, const double* grad_out, double* grad_a, double* grad_b) {
+  return pairwise_backward(ctx, A, B, use_mass, grad_out, grad_a, grad_b, false);
+}
+
+int rmsd_pairwise_backward_f32(rmsd_ctx* ctx, const rmsd_frames* A, const rmsd_frames* B,
+                               int use_mass, const float* grad_out, float* grad_a, float* grad_b) {
+  return pairwise_backward(ctx, A, B, use_mass, grad_out, grad_a, grad_b, true);
 }
 
 }  // extern "C"

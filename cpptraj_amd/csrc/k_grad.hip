@@ -59,13 +59,36 @@ __global__ __launch_bounds__(256) void k_fit_grad(FrameSetDev fs, const double* 
   g[2] = (G)(s * (x2 - u2));
 }
 
-// Centred FP64 coordinates, SoA [F][3][n], and sum w |x~|^2 per frame.
-__global__ __launch_bounds__(256) void k_center(FrameSetDev fs, const double* w, double* xc,
-                                                double* g) {
+// Centred FP64 coordinates, SoA [F][3][n], and sum w |x~|^2 per frame, of both
+// sets, and the total weight: the frames of A, then of B, one workgroup each,
+// then one workgroup for the weight's chain of additions (35 us in front of the
+// others when it had a launch of its own, at 2,000 weights).
+constexpr int CENTER_STAGE = 512;
+struct CenterArgs {
+  FrameSetDev A, B;
+  const double* w;
+  double* xa;
+  double* xb;
+  double* ga;
+  double* gb;
+  double* W;
+};
+
+__global__ __launch_bounds__(256) void k_center(CenterArgs a) {
   __shared__ double red[4 * 4];
-  const int64_t f = blockIdx.x;
-  const int n = fs.nsel;
+  __shared__ double stage[CENTER_STAGE];
+  const int n = a.A.nsel;
+  int64_t f = blockIdx.x;
+  if (f == (int64_t)a.A.nframes + a.B.nframes) {
+    rmsd_dev::mass_chain<CENTER_STAGE>(a.w, n, n, nullptr, stage, a.W);
+    return;
+  }
+  const bool first = f < a.A.nframes;
+  if (!first) f -= a.A.nframes;
+  const FrameSetDev& fs = first ? a.A : a.B;
+  const double* w = a.w;
   double v[4] = {0, 0, 0, 0};
+#pragma unroll 4
   for (int k = threadIdx.x; k < n; k += blockDim.x) {
     const double m = w ? w[k] : 1.0;
     float p[3];
@@ -80,7 +103,8 @@ __global__ __launch_bounds__(256) void k_center(FrameSetDev fs, const double* w,
   const double inv = tot != 0.0 ? 1.0 / tot : 0.0;
   const double c0 = v[0] * inv, c1 = v[1] * inv, c2 = v[2] * inv;
   double e[1] = {0.0};
-  double* out = xc + f * 3 * n;
+  double* out = (first ? a.xa : a.xb) + f * 3 * n;
+#pragma unroll 4
   for (int k = threadIdx.x; k < n; k += blockDim.x) {
     float p[3];
     load_atom(fs, f, k, p);
@@ -93,7 +117,7 @@ __global__ __launch_bounds__(256) void k_center(FrameSetDev fs, const double* w,
     e[0] += (w ? w[k] : 1.0) * (x0 * x0 + x1 * x1 + x2 * x2);
   }
   rmsd_dev::block_sum<1>(e, red);
-  if (threadIdx.x == 0) g[f] = e[0];
+  if (threadIdx.x == 0) (first ? a.ga : a.gb)[f] = e[0];
 }
 
 // One workgroup per 16 x 16 block of pairs (i target, j reference);
@@ -104,17 +128,19 @@ __global__ __launch_bounds__(256) void k_center(FrameSetDev fs, const double* w,
 // s = 0..3, of row frame i0 + l % 16 (A, 16 x 4) and of column frame j0 + l % 16
 // (B, 4 x 16), four consecutive atoms of a coordinate row (two 16-byte loads
 // when n is even).  The four waves take a quarter of the atoms each; their
-// partial sums are added in a fixed order through LDS, and wave 0 solves the
-// block's pairs: FP64 QCP, rotation, c_ij.  (One thread per pair with a serial
-// atom loop took 6.2 ms for 512 x 512 pairs of 2,000 atoms; one wave per block
-// over all atoms 0.58 ms.)
+// partial sums are exchanged through LDS and added in a fixed order, item v of
+// the accumulators by wave v, which solves those pairs: FP64 QCP, rotation,
+// c_ij (a pair per lane).  512 x 512 pairs of 2,000 atoms: 0.24 ms (40 TFLOP/s),
+// as with every pair solved by wave 0, four per lane, or with the next step's
+// atoms prefetched: 1.6 GB of operands from beyond L2 bound it.
 typedef __attribute__((ext_vector_type(4))) double f64x4_g;
 typedef __attribute__((ext_vector_type(2))) double f64x2_g;
 constexpr int ROT_SPLIT = 4;
+template <class GT>
 __global__ __launch_bounds__(64 * ROT_SPLIT) __attribute__((amdgpu_waves_per_eu(2))) void k_pair_rot(
     const double* XA, const double* XB, const double* gA, const double* gB, const double* w, int n,
-    int FA, int FB, const double* Mp, const double* G, double* cw) {
-  __shared__ double part[2][36][64];
+    int FA, int FB, const double* Mp, const GT* G, double* cw) {
+  __shared__ double part[ROT_SPLIT][3][9][64];  // [reader][the others][element][lane]
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int nbj = (FB + 15) / 16;
   const int64_t blk = blockIdx.x;  // the grid is the block count: no workgroup exits early
@@ -180,33 +206,29 @@ __global__ __launch_bounds__(64 * ROT_SPLIT) __attribute__((amdgpu_waves_per_eu(
         for (int d = 0; d < 3; ++d)
           acc[c][d] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[s4][c], bv[s4][d], acc[c][d], 0, 0, 0);
   }
-  // (acc0 + acc2) + (acc1 + acc3), in that order
-  if (wave >= 2)
+  // Wave v takes item v of every wave's accumulators: its own, and those of the
+  // others in the slots of their order.
 #pragma unroll
-    for (int e = 0; e < 36; ++e) part[wave - 2][e][lane] = acc[e / 12][(e / 4) % 3][e % 4];
+  for (int v = 0; v < ROT_SPLIT; ++v)
+    if (v != wave)
+#pragma unroll
+      for (int e = 0; e < 9; ++e) part[v][wave < v ? wave : wave - 1][e][lane] = acc[e / 3][e % 3][v];
   __syncthreads();
-  if (wave < 2)
+  double S[9];
 #pragma unroll
-    for (int e = 0; e < 36; ++e) acc[e / 12][(e / 4) % 3][e % 4] += part[wave][e][lane];
-  __syncthreads();
-  if (wave == 1)
+  for (int e = 0; e < 9; ++e) {
+    const f64x4_g& x4 = acc[e / 3][e % 3];
+    const double own = wave == 0 ? x4[0] : wave == 1 ? x4[1] : wave == 2 ? x4[2] : x4[3];
+    double s[ROT_SPLIT];
 #pragma unroll
-    for (int e = 0; e < 36; ++e) part[0][e][lane] = acc[e / 12][(e / 4) % 3][e % 4];
-  __syncthreads();
-  if (wave != 0) return;
-#pragma unroll
-  for (int e = 0; e < 36; ++e) acc[e / 12][(e / 4) % 3][e % 4] += part[0][e][lane];
+    for (int u = 0; u < ROT_SPLIT; ++u)
+      s[u] = u == wave ? own : part[wave][u < wave ? u : u - (u > 0)][e][lane];
+    S[e] = (s[0] + s[2]) + (s[1] + s[3]);
+  }
   const double M = Mp[0];
   // The accumulators hold row (lane / 16) + 4 v, column lane % 16, in item v.
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    const int64_t i = i0 + (lane >> 4) + 4 * v, j = fj;
-    if (i >= FA || !jok) continue;
-    double S[9];
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-#pragma unroll
-      for (int d = 0; d < 3; ++d) S[3 * c + d] = acc[c][d][v];
+  const int64_t i = i0 + (lane >> 4) + 4 * wave, j = fj;
+  if (i < FA && jok) {
     const int64_t p = i * FB + j;
     const double E0 = 0.5 * (gA[i] + gB[j]);
     const rmsd_dev::QcpCoef co = rmsd_dev::qcp_coefficients(S);
@@ -214,7 +236,7 @@ __global__ __launch_bounds__(64 * ROT_SPLIT) __attribute__((amdgpu_waves_per_eu(
     const double r = rmsd_dev::rmsd_from_lambda(E0, lam, M, 1);
     double U[9];
     rmsd_dev::qcp_rotation(S, lam, U);
-    const double cc = (r > 1e-12) ? G[p] / r : 0.0;
+    const double cc = (r > 1e-12) ? (double)G[p] / r : 0.0;
     double* o = cw + p * 10;
     o[0] = cc;
     for (int k = 0; k < 9; ++k) o[1 + k] = cc * U[k];
@@ -226,64 +248,94 @@ __global__ __launch_bounds__(64 * ROT_SPLIT) __attribute__((amdgpu_waves_per_eu(
 //   ROWS (own i, partners j):     O[i][c][k] = sum_j sum_b (c U)_ij[b][c] y~_j[b][k]
 //   columns (own j, partners i):  O[j][c][k] = sum_i sum_a (c U)_ij[c][a] x~_i[a][k]
 //   grad[o][k][c] = w_k / M (cs_o own~_o[c][k] - O[o][c][k]),  cs_o = sum_p c_op.
-// One wave per 16 own frames x 32 atoms.  Per step of 4 partners, lane l holds
-// the pair record (c, c U) of own frame o0 + l % 16 and partner p0 + l / 16
-// (five 16-byte loads): the A operands (16 x 4) of the nine (own coordinate,
-// partner coordinate) products; B (4 x 16) is the partner's coordinate row at
-// atoms k0 + 16 g + l % 16.  (A thread per atom with the coefficients of one
-// partner per LDS stage: 0.58 ms per side for 512 x 512 pairs of 2,000 atoms.)
-constexpr int GKT = 2;  // 16-atom tiles per wave (4: 0.97 ms, 1: 0.90 ms for the whole call)
-template <bool ROWS>
-__global__ __launch_bounds__(256) void k_grad_sum(const double* XA, const double* XB,
-                                                  const double* cw, const double* w, int n, int FA,
-                                                  int FB, const double* Mp, double* grad) {
-  const int lane = threadIdx.x & 63;
+// A workgroup takes 16 own frames and 128 atoms, 32 per wave, and both sides run
+// in one launch (rows first).  The pair records (c, c U) of 16 partners at a time
+// go to LDS, one record (80 contiguous bytes) per thread, the next 16 in flight
+// meanwhile, and serve the four waves: lane l's A operand (16 x 4) is the record
+// of own frame o0 + l % 16 and partner p0 + 4 s + l / 16, for nine (own
+// coordinate, partner coordinate) products; B (4 x 16) is the partner's
+// coordinate row at atoms k0 + 16 g + l % 16, loaded a step ahead.  Bound by FP64
+// MFMA: 512 x 512 pairs of 2,000 atoms, both sides 0.35 ms (54 TFLOP/s).  Each wave
+// reading its own records, five 16-byte loads strided by the partner rows per 18
+// MFMAs, took 0.27 + 0.24 ms, 1.3 GB of records a side from L2.
+constexpr int GKT = 2;         // 16-atom tiles per wave
+constexpr int GATOMS = 64 * GKT;  // atoms per workgroup
+constexpr int GPART = 16;      // partners per LDS stage
+constexpr int GLD = 17;        // own frames' row in LDS, padded
+
+template <bool ROWS, class T>
+__device__ __forceinline__ void grad_sum_body(const double* XA, const double* XB, const double* cw,
+                                              const double* w, int n, int FA, int FB,
+                                              const double* Mp, T* grad, int blk,
+                                              double (*rec)[GPART * GLD]) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int NO = ROWS ? FA : FB, NP = ROWS ? FB : FA;  // own frames, partners
   const double* XO = ROWS ? XA : XB;
   const double* XP = ROWS ? XB : XA;
-  const int nkt = (n + 16 * GKT - 1) / (16 * GKT);
-  const int64_t wv = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (wv >= (int64_t)((NO + 15) / 16) * nkt) return;  // whole waves; no barriers here
-  const int o0 = (int)(wv / nkt) * 16, k0 = (int)(wv % nkt) * 16 * GKT;
-  const int ol = o0 + (lane & 15);
-  const bool ook = ol < NO;
+  const int nkt = (n + GATOMS - 1) / GATOMS;
+  const int o0 = blk / nkt * 16, k0 = blk % nkt * GATOMS + wave * 16 * GKT;
+  // The record this thread stages: consecutive threads along the pairs' rows.
+  const int so = ROWS ? threadIdx.x >> 4 : threadIdx.x & 15;
+  const int sp = ROWS ? threadIdx.x & 15 : threadIdx.x >> 4;
+  f64x2_g nxt[5];
+  auto fetch = [&](int p0) {
+    const int o = o0 + so, p = p0 + sp;
+#pragma unroll
+    for (int t = 0; t < 5; ++t) nxt[t] = f64x2_g{0.0, 0.0};
+    if (o < NO && p < NP) {
+      const int64_t pair = ROWS ? (int64_t)o * FB + p : (int64_t)p * FB + o;
+      const f64x2_g* r2 = reinterpret_cast<const f64x2_g*>(cw + pair * 10);
+#pragma unroll
+      for (int t = 0; t < 5; ++t) nxt[t] = r2[t];
+    }
+  };
+  double bn[GKT][3];
+  auto partner = [&](int p) {  // the B operands of partners p ... p + 3
+    const int pl = p + (lane >> 4);
+    const double* yp = XP + (int64_t)(pl < NP ? pl : 0) * 3 * n;
+#pragma unroll
+    for (int g = 0; g < GKT; ++g) {
+      const int k = k0 + 16 * g + (lane & 15);
+#pragma unroll
+      for (int b = 0; b < 3; ++b) bn[g][b] = pl < NP && k < n ? yp[(int64_t)b * n + k] : 0.0;
+    }
+  };
   f64x4_g acc[GKT][3];
 #pragma unroll
   for (int g = 0; g < GKT; ++g)
 #pragma unroll
     for (int c = 0; c < 3; ++c) acc[g][c] = f64x4_g{0.0, 0.0, 0.0, 0.0};
   double csum = 0.0;
-  for (int p0 = 0; p0 < NP; p0 += 4) {
-    const int pl = p0 + (lane >> 4);
-    const bool pok = pl < NP;
-    double rec[10];
+  fetch(0);
+  partner(0);
+  for (int p0 = 0; p0 < NP; p0 += GPART) {
+    __syncthreads();  // the last stage's reads
 #pragma unroll
-    for (int t = 0; t < 10; ++t) rec[t] = 0.0;
-    if (ook && pok) {
-      const int64_t pair = ROWS ? (int64_t)ol * FB + pl : (int64_t)pl * FB + ol;
-      const f64x2_g* r2 = reinterpret_cast<const f64x2_g*>(cw + pair * 10);
-#pragma unroll
-      for (int t = 0; t < 5; ++t) {
-        const f64x2_g v = r2[t];
-        rec[2 * t] = v.x;
-        rec[2 * t + 1] = v.y;
-      }
+    for (int t = 0; t < 5; ++t) {
+      rec[2 * t][sp * GLD + so] = nxt[t].x;
+      rec[2 * t + 1][sp * GLD + so] = nxt[t].y;
     }
-    csum += rec[0];
-    const double* yp = XP + (int64_t)(pok ? pl : 0) * 3 * n;
+    __syncthreads();
+    fetch(p0 + GPART);
 #pragma unroll
-    for (int g = 0; g < GKT; ++g) {
-      const int k = k0 + 16 * g + (lane & 15);
-      double bv[3] = {0.0, 0.0, 0.0};
-      if (pok && k < n)
+    for (int s = 0; s < GPART / 4; ++s) {
+      double bv[GKT][3];
 #pragma unroll
-        for (int b = 0; b < 3; ++b) bv[b] = yp[b * n + k];
+      for (int g = 0; g < GKT; ++g)
+#pragma unroll
+        for (int b = 0; b < 3; ++b) bv[g][b] = bn[g][b];
+      partner(p0 + 4 * s + 4);
+      const int at = (4 * s + (lane >> 4)) * GLD + (lane & 15);
+      csum += rec[0][at];
 #pragma unroll
       for (int c = 0; c < 3; ++c)
 #pragma unroll
-        for (int b = 0; b < 3; ++b)
-          acc[g][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(ROWS ? rec[1 + 3 * b + c] : rec[1 + 3 * c + b],
-                                                           bv[b], acc[g][c], 0, 0, 0);
+        for (int b = 0; b < 3; ++b) {
+          const double av = rec[ROWS ? 1 + 3 * b + c : 1 + 3 * c + b][at];
+#pragma unroll
+          for (int g = 0; g < GKT; ++g)
+            acc[g][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv[g][b], acc[g][c], 0, 0, 0);
+        }
     }
   }
   // cs of own frame o0 + r: lanes r, r + 16, r + 32, r + 48
@@ -302,11 +354,41 @@ __global__ __launch_bounds__(256) void k_grad_sum(const double* XA, const double
       const int k = k0 + 16 * g + (lane & 15);
       if (k >= n) continue;
       const double s = (w ? w[k] : 1.0) / M;
-      double* gp_ = grad + ((int64_t)o * n + k) * 3;
+      T* gp_ = grad + ((int64_t)o * n + k) * 3;
 #pragma unroll
-      for (int c = 0; c < 3; ++c) gp_[c] = s * (cs * xo[c * n + k] - acc[g][c][v]);
+      for (int c = 0; c < 3; ++c) gp_[c] = (T)(s * (cs * xo[(int64_t)c * n + k] - acc[g][c][v]));
     }
   }
+}
+
+template <class T>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_grad_sum(
+    const double* XA, const double* XB, const double* cw, const double* w, int n, int FA, int FB,
+    const double* Mp, T* gradA, T* gradB, int nrows) {
+  __shared__ double rec[10][GPART * GLD];
+  if ((int)blockIdx.x < nrows)
+    grad_sum_body<true>(XA, XB, cw, w, n, FA, FB, Mp, gradA, blockIdx.x, rec);
+  else
+    grad_sum_body<false>(XA, XB, cw, w, n, FA, FB, Mp, gradB, blockIdx.x - nrows, rec);
+}
+
+template <class GT, class T>
+hipError_t pair_grad(const double* XA, const double* XB, const double* gA, const double* gB,
+                     const double* w, int n, int FA, int FB, const double* M, const GT* G,
+                     double* cw, T* gradA, T* gradB, hipStream_t s) {
+  const int64_t nblk = (int64_t)((FA + 15) / 16) * ((FB + 15) / 16);
+  if (nblk > 0x7fffffff) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_pair_rot<GT>, dim3((unsigned)nblk), dim3(64 * ROT_SPLIT), 0, s, XA, XB, gA,
+                     gB, w, n, FA, FB, M, G, cw);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  const int64_t nkt = (n + GATOMS - 1) / GATOMS;
+  const int64_t rows = gradA ? (FA + 15) / 16 * nkt : 0, cols = gradB ? (FB + 15) / 16 * nkt : 0;
+  if (rows + cols > 0x7fffffff) return hipErrorInvalidValue;
+  if (rows + cols > 0)
+    hipLaunchKernelGGL(k_grad_sum<T>, dim3((unsigned)(rows + cols)), dim3(256), 0, s, XA, XB, cw, w, n,
+                       FA, FB, M, gradA, gradB, (int)rows);
+  return hipGetLastError();
 }
 
 }  // namespace
@@ -325,34 +407,21 @@ hipError_t rmsd_launch_fit_grad(const FrameSetDev& fs, const double* mass, const
   return hipGetLastError();
 }
 
-hipError_t rmsd_launch_center(const FrameSetDev& fs, const double* w, double* xc, double* g,
-                              hipStream_t s) {
-  hipLaunchKernelGGL(k_center, dim3(fs.nframes), dim3(256), 0, s, fs, w, xc, g);
+hipError_t rmsd_launch_center(const FrameSetDev& A, const FrameSetDev& B, const double* w, double* xa,
+                              double* xb, double* ga, double* gb, double* W, hipStream_t s) {
+  const int64_t grid = (int64_t)A.nframes + B.nframes + 1;
+  if (grid > 0x7fffffff) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_center, dim3((unsigned)grid), dim3(256), 0, s,
+                     CenterArgs{A, B, w, xa, xb, ga, gb, W});
   return hipGetLastError();
 }
 
 hipError_t rmsd_launch_pair_grad(const double* XA, const double* XB, const double* gA,
                                  const double* gB, const double* w, int n, int FA, int FB,
-                                 const double* M, const double* G, double* cw, double* gradA,
-                                 double* gradB, hipStream_t s) {
-  const int64_t nblk = (int64_t)((FA + 15) / 16) * ((FB + 15) / 16);
-  if (nblk > 0x7fffffff) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_pair_rot, dim3((unsigned)nblk), dim3(64 * ROT_SPLIT), 0, s, XA, XB, gA, gB,
-                     w, n, FA, FB, M, G, cw);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  const int nkt = (n + 16 * GKT - 1) / (16 * GKT);
-  if (gradA) {
-    const int64_t waves = (int64_t)((FA + 15) / 16) * nkt;
-    hipLaunchKernelGGL(k_grad_sum<true>, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, s, XA, XB,
-                       cw, w, n, FA, FB, M, gradA);
-    if ((e = hipGetLastError()) != hipSuccess) return e;
-  }
-  if (gradB) {
-    const int64_t waves = (int64_t)((FB + 15) / 16) * nkt;
-    hipLaunchKernelGGL(k_grad_sum<false>, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, s, XA, XB,
-                       cw, w, n, FA, FB, M, gradB);
-    e = hipGetLastError();
-  }
-  return e;
+                                 const double* M, const void* G, double* cw, void* gradA,
+                                 void* gradB, bool f32, hipStream_t s) {
+  return f32 ? pair_grad(XA, XB, gA, gB, w, n, FA, FB, M, static_cast<const float*>(G), cw,
+                         static_cast<float*>(gradA), static_cast<float*>(gradB), s)
+             : pair_grad(XA, XB, gA, gB, w, n, FA, FB, M, static_cast<const double*>(G), cw,
+                         static_cast<double*>(gradA), static_cast<double*>(gradB), s);
 }

@@ -720,26 +720,31 @@ __global__ __launch_bounds__(64 * NWR * NWC) void k_pairwise(PairArgs args) {
   pair_tile<PREC, WR, WC, NWR, NWC>(args, args.tiles[t], t);
 }
 
-// FP64, single matrix: a workgroup of one wave takes a 16 x 16 block of the
-// pairs of a 64 x 64 tile of the list.  Blocks this small fill the chip from a
-// few hundred frames on (64 x 64 workgroups left 192 of 256 CUs idle at 512 x
-// 512 pairs, and CUs idle in the last round of a few), skip the empty half of
-// the diagonal's tiles, and run three to a SIMD (<= 168 registers), so that one
-// wave's FP64 solves run beside the others' MFMAs.  Bound by FP64 MFMA: 3,001 x
-// 305 429 us (58 TFLOP/s with the preparation) against 489 in eight-wave 64 x 64
-// workgroups of 16 x 32 blocks, 512 frames x 2,000 185 / 586, 101 x 66 14.2 /
-// 35.6, 1,000 x 2,000 457 / 593, 8,000 x 1,200 10.4 / 10.6 ms.  Left to choose
-// its registers the compiler takes 200, two waves per SIMD: 566 us at 3,001 x 305.
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_pairwise_f64(
+// FP64, single matrix: waves of one 16 x 16 block of the pairs of a 64 x 64 tile
+// of the list each, NW x NW of them to a workgroup.  Blocks this small fill the
+// chip from a few hundred frames on (64 x 64 workgroups left 192 of 256 CUs idle
+// at 512 x 512 pairs, and CUs idle in the last round of a few), skip the empty
+// half of the diagonal's tiles, and run three or more to a SIMD (<= 168
+// registers), so that one wave's FP64 solves run beside the others' MFMAs.  Bound
+// by FP64 MFMA: 3,001 x 305 429 us (58 TFLOP/s with the preparation) against 489
+// in eight-wave 64 x 64 workgroups of 16 x 32 blocks, 512 frames x 2,000 171 /
+// 586, 101 x 66 14.2 / 35.6, 1,000 x 2,000 445 / 593, 8,000 x 1,200 10.4 / 10.6
+// ms.  Left to choose its registers the compiler takes 200, two waves per SIMD:
+// 566 us at 3,001 x 305.
+template <int NW>
+__global__ __launch_bounds__(64 * NW * NW) __attribute__((amdgpu_waves_per_eu(3))) void k_pairwise_f64(
     PairArgs args) {
+  constexpr int PC = 4 / NW, PARTS = PC * PC;  // workgroups of a tile
   const int i = blockIdx.x / args.nxcd;
-  const int t = (blockIdx.x % args.nxcd) * args.per_xcd + i / 16;
+  const int t = (blockIdx.x % args.nxcd) * args.per_xcd + i / PARTS;
   if (t >= args.ntiles) return;
   const int2 tile = args.tiles[t];
-  const int64_t fbA = (int64_t)tile.x * 4 + i % 16 / 4, fbB = (int64_t)tile.y * 4 + i % 4;
+  const int wave = threadIdx.x >> 6;
+  const int64_t fbA = (int64_t)tile.x * 4 + i % PARTS / PC * NW + wave / NW;
+  const int64_t fbB = (int64_t)tile.y * 4 + i % PC * NW + wave % NW;
   if (fbA * 16 >= args.FA || fbB * 16 >= args.FB) return;
   if (args.tri && fbA > fbB) return;  // no pair above the diagonal
-  pair_block<PREC_F64, 1, 1>(args, fbA, fbB, t, 0, 1);
+  pair_block<PREC_F64, 1, 1>(args, fbA, fbB, t, wave, NW * NW);
 }
 
 // ---- batched matrices ---------------------------------------------------------------
@@ -863,16 +868,23 @@ static hipError_t launch_shared(const PairArgs& a, hipStream_t s) {
   return hipGetLastError();
 }
 
+// Four waves to a workgroup while there are few blocks per SIMD: a workgroup's
+// waves go to the four SIMDs of a CU, where single waves were seen to share a
+// SIMD beside idle ones (1,024 blocks of 2,000 atoms on 1,024 SIMDs: 302 us
+// against 172).  One wave beyond (1 to 2 % faster: nothing waits for a
+// workgroup's last wave).
+constexpr int F64_QUAD_TILES = 1024;
+template <int NW>
 static hipError_t launch_f64(const PairArgs& a, hipStream_t s) {
-  const int64_t grid = (int64_t)a.per_xcd * a.nxcd * 16;
+  const int64_t grid = (int64_t)a.per_xcd * a.nxcd * (16 / (NW * NW));
   if (grid > 0x7fffffff) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_pairwise_f64, dim3((unsigned)grid), dim3(64), 0, s, a);
+  hipLaunchKernelGGL(k_pairwise_f64<NW>, dim3((unsigned)grid), dim3(64 * NW * NW), 0, s, a);
   return hipGetLastError();
 }
 
 hipError_t rmsd_launch_pairwise(int prec, const PairArgs& a, hipStream_t s) {
   switch (prec) {
-    case PREC_F64: return launch_f64(a, s);
+    case PREC_F64: return a.ntiles <= F64_QUAD_TILES ? launch_f64<2>(a, s) : launch_f64<1>(a, s);
     case PREC_F32: return launch_tiles<PREC_F32, 2, 3, 2, 2>(a, s);
     case PREC_BF16X3: return launch_shared<PREC_BF16X3>(a, s);
     default: return hipErrorInvalidValue;

@@ -27,6 +27,12 @@
 namespace {
 
 constexpr int PREP_THREADS = 64;
+// FP64: few frames, or fewer than a chip's fill of larger ones, take four waves
+// each (512 x 2,000: 42 -> 20 us; 101 x 66 1.3 us faster, 1,500 x 66 2.7 us slower
+// than single waves).
+constexpr bool prep_wide(int frames, int atoms) {
+  return frames <= 512 || (frames < 8192 && atoms > 256);
+}
 
 template <int PREC>
 __device__ __forceinline__ int64_t packed_elem(int64_t f, int k, int c, int p, int KB) {
@@ -263,58 +269,131 @@ __global__ __launch_bounds__(PREP_THREADS) void k_setup_batch(const SetupArgs* s
 }
 
 // ---- per-frame preparation -----------------------------------------------------
+// Padding frames: zero operands so that padded rows and columns of a tile
+// contribute nothing.
+template <int PREC>
+__device__ __forceinline__ void prep_padding(const PrepArgs& a, int64_t f) {
+  if (a.nrm && threadIdx.x < 4) gp(a.nrm)[4 * f + threadIdx.x] = 0.0;
+  if (a.cen && threadIdx.x < 4) gp(a.cen)[4 * f + threadIdx.x] = 0.0;
+  for (int k = threadIdx.x; k < a.Kp; k += blockDim.x)
+    for (int c = 0; c < 3; ++c)
+      for (int p = 0; p < chunk_parts(PREC); ++p) {
+        const int64_t e = packed_elem<PREC>(f, k, c, p, a.KB);
+        if (PREC == PREC_F64) gp(reinterpret_cast<double*>(a.packed))[e] = 0.0;
+        else if (PREC == PREC_F32) gp(reinterpret_cast<float*>(a.packed))[e] = 0.0f;
+        else gp(reinterpret_cast<__bf16*>(a.packed))[e] = (__bf16)0.0f;
+      }
+}
+
+// FP64: one frame by one wave, or by four where few frames leave the chip idle
+// (THREADS 64 or 256), to the same bits: atoms k with k / 64 = c (mod 4) form
+// partial sum c, held by lane k % 64 of the one wave or of wave c, and the four
+// are added in order.  512 frames x 2,000 weighted atoms: 42 us by single waves
+// with one running sum.
+template <int NV, int THREADS>
+__device__ __forceinline__ void quarter_sums(const double (&v)[THREADS == 64 ? 4 : 1][NV],
+                                             double* red, double (&tot)[NV]) {
+  if constexpr (THREADS == 64) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      tot[i] = rmsd_dev::wave_sum(v[0][i]);
+#pragma unroll
+      for (int c = 1; c < 4; ++c) tot[i] += rmsd_dev::wave_sum(v[c][i]);
+    }
+  } else {
+    const int wave = threadIdx.x >> 6;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const double s = rmsd_dev::wave_sum(v[0][i]);
+      if ((threadIdx.x & 63) == 0) red[wave * NV + i] = s;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      tot[i] = red[i];
+#pragma unroll
+      for (int c = 1; c < 4; ++c) tot[i] += red[c * NV + i];
+    }
+    __syncthreads();
+  }
+}
+
+template <int THREADS>
+__device__ __forceinline__ void prep_f64(const PrepArgs& a, int64_t f) {
+#pragma clang fp contract(on)
+  __shared__ double red[16];
+  constexpr int NC = THREADS == 64 ? 4 : 1;
+  const int n = a.fs.nsel;
+  double v[NC][4];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) v[c][0] = v[c][1] = v[c][2] = v[c][3] = 0.0;
+  for (int k0 = 0; k0 < n; k0 += 256)
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int k = k0 + 64 * c + threadIdx.x;
+      if (k < n) {
+        const double m = a.cmass ? gp(a.cmass)[k] : 1.0;
+        float p[3];
+        load_atom(a.fs, f, k, p);
+        v[c][0] += m * (double)p[0];
+        v[c][1] += m * (double)p[1];
+        v[c][2] += m * (double)p[2];
+        v[c][3] += m;
+      }
+    }
+  double s[4];
+  quarter_sums<4, THREADS>(v, red, s);
+  const double tot = a.cmass ? s[3] : (double)n;
+  const double inv = tot != 0.0 ? 1.0 / tot : 0.0;
+  const double cen[3] = {s[0] * inv, s[1] * inv, s[2] * inv};
+  if (a.cen && threadIdx.x == 0) {
+    gp(a.cen)[4 * f] = cen[0];
+    gp(a.cen)[4 * f + 1] = cen[1];
+    gp(a.cen)[4 * f + 2] = cen[2];
+    gp(a.cen)[4 * f + 3] = 0.0;
+  }
+  double g[NC][1];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) g[c][0] = 0.0;
+  const auto out = gp(reinterpret_cast<double*>(a.packed));
+  for (int k0 = 0; k0 < a.Kp; k0 += 256)
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int k = k0 + 64 * c + threadIdx.x;
+      if (k < a.Kp) {
+        double x[3];
+        centred(a.fs, f, k, cen, a.smass, x);
+#pragma unroll
+        for (int d = 0; d < 3; ++d) out[packed_elem<PREC_F64>(f, k, d, 0, a.KB)] = x[d];
+        g[c][0] += x[0] * x[0] + x[1] * x[1] + x[2] * x[2];
+      }
+    }
+  double G[1];
+  quarter_sums<1, THREADS>(g, red, G);
+  if (threadIdx.x == 0) gp(a.g)[f] = G[0];
+}
+
 // QUADS = false compiles the atom-by-atom path only (fewer registers and no
 // branch to the quad code: the batched launch for sets without quads).
 template <int PREC, bool QUADS = true>
 __device__ __forceinline__ void prep_body(const PrepArgs& a, int64_t f) {
-  __shared__ double red[24 * (PREP_THREADS / 64)];
   const int Kp = a.Kp;
-
   if (f >= a.fs.nframes) {
-    // Padding frames: zero operands so that padded rows and columns of a tile
-    // contribute nothing.
-    if (a.nrm && threadIdx.x < 4) gp(a.nrm)[4 * f + threadIdx.x] = 0.0;
-    if (a.cen && threadIdx.x < 4) gp(a.cen)[4 * f + threadIdx.x] = 0.0;
-    for (int k = threadIdx.x; k < Kp; k += blockDim.x)
-      for (int c = 0; c < 3; ++c)
-        for (int p = 0; p < chunk_parts(PREC); ++p) {
-          const int64_t e = packed_elem<PREC>(f, k, c, p, a.KB);
-          if (PREC == PREC_F64) gp(reinterpret_cast<double*>(a.packed))[e] = 0.0;
-          else if (PREC == PREC_F32) gp(reinterpret_cast<float*>(a.packed))[e] = 0.0f;
-          else gp(reinterpret_cast<__bf16*>(a.packed))[e] = (__bf16)0.0f;
-        }
+    prep_padding<PREC>(a, f);
     return;
   }
+  if constexpr (PREC == PREC_F64) {
+    prep_f64<PREP_THREADS>(a, f);
+    return;
+  } else {
+  __shared__ double red[24 * (PREP_THREADS / 64)];
 
   // MFMA forms on frames that allow 16-byte loads of four atoms: each lane
   // takes quads of atoms (four per step; the 50,000 x 1,200 AoS stage: 1.05 ->
   // 0.86 ms).  Otherwise lanes take consecutive atoms (coalesced 4-byte loads;
   // quads of such atoms would spread each load over four times the lines).
-  const int lay = PREC == PREC_F64 || !QUADS ? 0 : quad_layout(a.fs);
+  const int lay = !QUADS ? 0 : quad_layout(a.fs);
   double cen[3];
-  if (PREC == PREC_F64) {
-    centroid(a.fs, f, a.cmass, red, cen);
-    if (a.cen && threadIdx.x == 0) {
-      gp(a.cen)[4 * f] = cen[0];
-      gp(a.cen)[4 * f + 1] = cen[1];
-      gp(a.cen)[4 * f + 2] = cen[2];
-      gp(a.cen)[4 * f + 3] = 0.0;
-    }
-    double g[1] = {0.0};
-    const auto out = gp(reinterpret_cast<double*>(a.packed));
-    for (int k = threadIdx.x; k < Kp; k += blockDim.x) {
-      double x[3];
-      centred(a.fs, f, k, cen, a.smass, x);
-      out[packed_elem<PREC>(f, k, 0, 0, a.KB)] = x[0];
-      out[packed_elem<PREC>(f, k, 1, 0, a.KB)] = x[1];
-      out[packed_elem<PREC>(f, k, 2, 0, a.KB)] = x[2];
-      g[0] += x[0] * x[0] + x[1] * x[1] + x[2] * x[2];
-    }
-    rmsd_dev::block_sum<1>(g, red);
-    if (threadIdx.x == 0) gp(a.g)[f] = g[0];
-    return;
-  }
-
   // MFMA-reduced forms: align to the template in FP64.  One pass over the
   // frame gives the centroid and the moments about the origin: with s = sqrt(w)
   // the fit weights and c the centroid,
@@ -520,6 +599,7 @@ __device__ __forceinline__ void prep_body(const PrepArgs& a, int64_t f) {
       gp(a.nrm)[4 * f + 3] = sqrt(l2);
     }
   }
+  }  // MFMA-reduced forms
 }
 
 // Workgroup -> frame.  The hardware deals consecutive workgroups round-robin
@@ -541,9 +621,15 @@ int64_t prep_grid(int64_t n) {
 
 template <int PREC>
 __global__ __launch_bounds__(PREP_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void k_prep(PrepArgs a) {
-  if (PREC == PREC_F64 && a.wsum && blockIdx.x == gridDim.x - 1) {
-    // FP64 needs no template and the total weight only behind the contraction:
-    // one more workgroup here instead of a launch before.
+  const int64_t f = prep_frame(blockIdx.x);
+  if (f < a.Fp) prep_body<PREC>(a, f);
+}
+
+// FP64 needs no template, and the total weight only behind the contraction: it
+// is one more workgroup here instead of a launch before.
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void k_prep_f64(PrepArgs a) {
+  if (a.wsum && blockIdx.x == gridDim.x - 1) {
     SetupArgs w;
     w.fs = a.fs;
     w.smass = a.smass;
@@ -552,7 +638,9 @@ __global__ __launch_bounds__(PREP_THREADS) __attribute__((amdgpu_waves_per_eu(4)
     return;
   }
   const int64_t f = prep_frame(blockIdx.x);
-  if (f < a.Fp) prep_body<PREC>(a, f);
+  if (f >= a.Fp) return;
+  if (f >= a.fs.nframes) prep_padding<PREC_F64>(a, f);
+  else prep_f64<THREADS>(a, f);
 }
 
 // Every padded frame of every set of a batch in one launch: workgroup b is
@@ -644,8 +732,11 @@ hipError_t rmsd_launch_prep_batch(int prec, const PrepArgs* sets, const int* fba
 hipError_t rmsd_launch_prep(const PrepArgs& a, hipStream_t s) {
   switch (a.prec) {
     case PREC_F64:
-      hipLaunchKernelGGL(k_prep<PREC_F64>, dim3(prep_grid(a.Fp) + (a.wsum ? 1 : 0)),
-                         dim3(PREP_THREADS), 0, s, a);
+      if (prep_wide(a.Fp, a.fs.nsel))
+        hipLaunchKernelGGL(k_prep_f64<256>, dim3(prep_grid(a.Fp) + (a.wsum ? 1 : 0)), dim3(256), 0, s,
+                           a);
+      else
+        hipLaunchKernelGGL(k_prep_f64<64>, dim3(prep_grid(a.Fp) + (a.wsum ? 1 : 0)), dim3(64), 0, s, a);
       break;
     case PREC_F32:
       hipLaunchKernelGGL(k_prep<PREC_F32>, dim3(prep_grid(a.Fp)), dim3(PREP_THREADS), 0, s, a);

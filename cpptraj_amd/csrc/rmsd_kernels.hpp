@@ -469,12 +469,14 @@ hipError_t rmsd_launch_ref_prep(const FrameSetDev& fs, int f, const double* rmas
 hipError_t rmsd_launch_fit_grad(const FrameSetDev& fs, const double* mass, const double* ref,
                                 const double* xform, const double* rmsd, const double* gout,
                                 const double* consts, void* grad, bool f32, hipStream_t s);
-hipError_t rmsd_launch_center(const FrameSetDev& fs, const double* w, double* xc, double* g,
-                              hipStream_t s);
+// Both sets centred, their E0 halves, and W = sum w (A.nsel when null).
+hipError_t rmsd_launch_center(const FrameSetDev& A, const FrameSetDev& B, const double* w, double* xa,
+                              double* xb, double* ga, double* gb, double* W, hipStream_t s);
+// G, gradA, gradB: FP32 (f32) or FP64; the arithmetic is FP64.
 hipError_t rmsd_launch_pair_grad(const double* XA, const double* XB, const double* gA,
                                  const double* gB, const double* w, int n, int FA, int FB,
-                                 const double* M, const double* G, double* cw, double* gradA,
-                                 double* gradB, hipStream_t s);
+                                 const double* M, const void* G, double* cw, void* gradA,
+                                 void* gradB, bool f32, hipStream_t s);
 
 // Symmetry-corrected RMSD (k_symm.hip).  Group g owns entries goff[g] ..
 // goff[g+1] of gatoms (selection indices); pos[i] is atom i's entry or -1.

@@ -362,6 +362,10 @@ int rmsd_fit_backward_f32(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_f
 int rmsd_pairwise_backward(rmsd_ctx* ctx, const rmsd_frames* A, const rmsd_frames* B,
                            int use_mass, const double* grad_out, double* grad_a,
                            double* grad_b);
+/* The same from an FP32 grad_out (the precision of rmsd_pairwise's output),
+ * computed in FP64 and rounded to FP32 as it is stored. */
+int rmsd_pairwise_backward_f32(rmsd_ctx* ctx, const rmsd_frames* A, const rmsd_frames* B,
+                               int use_mass, const float* grad_out, float* grad_a, float* grad_b);
 
 /* Batched all-pairs matrices: many trajectories or masks, of uneven frame and
  * atom counts, in one launch of the contraction.  No single reference

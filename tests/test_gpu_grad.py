@@ -162,3 +162,33 @@ def test_fit_backward_in_registers(ctx, n, F):
     if n > 2:  # two atoms: the rotation is not unique
         rest = [f for f in range(F) if f != 1]
         assert np.abs(new[rest] - old[rest]).max() <= 1e-9 * np.abs(old[rest]).max()
+
+
+@pytest.mark.parametrize("FA,FB", [(1, 1), (1, 40), (16, 17), (33, 5), (20, 64)])
+@pytest.mark.parametrize("n,use_mass", [(3, False), (31, True), (128, False), (133, True), (514, True)])
+def test_pairwise_backward_edges(oracle, ctx, FA, FB, n, use_mass):
+    """The block gradient at the edges of its 16-frame blocks, partner stages,
+    atom tiles and weight stages against the oracle's gradient of one row and one
+    column, and its FP32 form against its FP64 one."""
+    import torch
+    from cpptraj_amd.autograd import _pairwise_backward, pairwise_backward
+    X = synth.noisy(n + FA, FA + FB, n, 0.8)
+    A, B = X[:FA], X[FA:]
+    m = synth.masses(np.random.default_rng(n), n)
+    G = np.random.default_rng(FB).normal(size=(FA, FB)).astype(np.float32)
+    ga, gb = pairwise_backward(dev(A), dev(B), dev(G).double(), dev(m), use_mass, ctx=ctx)
+    fa, fb = _pairwise_backward(dev(A), dev(B), dev(G), dev(m), use_mass, torch.float32, ctx=ctx)
+    assert torch.equal(fa, ga.float()) and torch.equal(fb, gb.float())
+    assert torch.isfinite(ga).all() and torch.isfinite(gb).all()
+    if n == 3:  # a plane: the two methods' rotations agree to ~1e-8 only
+        return
+    i, j = FA - 1, FB - 1
+    ei, ej = np.zeros((n, 3)), np.zeros((n, 3))
+    for q in range(FB):
+        ei += G[i, q] * oracle_target_grad(oracle, A[i].astype(np.float64),
+                                           B[q].astype(np.float64), m, use_mass)[1]
+    for q in range(FA):
+        ej += G[q, j] * oracle_target_grad(oracle, B[j].astype(np.float64),
+                                           A[q].astype(np.float64), m, use_mass)[1]
+    assert np.abs(ga[i].cpu().numpy() - ei).max() <= 1e-9 * np.abs(ei).max()
+    assert np.abs(gb[j].cpu().numpy() - ej).max() <= 1e-9 * np.abs(ej).max()
