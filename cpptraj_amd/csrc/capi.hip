@@ -820,7 +820,7 @@ int rmsd_transform(rmsd_ctx* ctx, const rmsd_frames* frames, const int32_t* atom
 }
 
 // Per-residue no-fit RMSD.  The residue table is validated here, cut into
-// pieces whose LDS image fits one workgroup, and uploaded as one blob:
+// pieces of one workgroup, and uploaded as one blob:
 //   res_off (nres+1 int) | tgt (L int) | ref (L int) | pieces (P int4) |
 //   tmass (L double) | rmass (L double)
 int rmsd_perres_nofit(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frames* ref,
@@ -862,54 +862,32 @@ int rmsd_perres_nofit(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frame
     if (ref_atoms[k] < 0 || ref_atoms[k] >= ref->natom)
       return fail(ctx, RMSD_ERR_ARG, "reference atom index out of range");
   }
-  // Pieces: runs of whole residues that fit PERRES_LDS_PIECE at one frame.  A
-  // piece stages its target atom span, or gathers its own atoms when the span
-  // is more than twice their number (lo = -1); a residue that would switch a
-  // run from one form to the other starts a new piece.
-  std::vector<int4> pieces;
-  auto staged = [](int span, int ne) { return span <= 2 * ne + 64 ? span : -1; };
-  for (int r = 0; r < nres;) {
-    int lo = INT32_MAX, hi = -1, r1 = r;
-    bool span_form = true;
-    while (r1 < nres) {
-      int l2 = lo, h2 = hi;
-      for (int k = res_off[r1]; k < res_off[r1 + 1]; ++k) {
-        l2 = std::min(l2, tgt_atoms[k]);
-        h2 = std::max(h2, tgt_atoms[k] + 1);
-      }
-      const int ne = res_off[r1 + 1] - res_off[r];
-      const int span = h2 > l2 ? h2 - l2 : 0;
-      const bool sf = staged(span, ne) >= 0;
-      const size_t b = rmsd_perres_lds_bytes(r1 + 1 - r, ne, sf ? span : ne, 1);
-      if (r1 > r && (b > PERRES_LDS_PIECE || sf != span_form || r1 - r >= PERRES_RES_PIECE))
-        break;
-      if (r1 == r && b > PERRES_LDS_MAX)
-        return fail(ctx, RMSD_ERR_ARG, "residue " + std::to_string(r) + " has too many atoms (" +
-                                           std::to_string(ne) + ") for per-residue RMSD");
-      lo = l2;
-      hi = h2;
-      span_form = sf;
-      ++r1;
+  // The largest residue: its atoms, and their span where that is at most twice
+  // their number, by rmsd_perres_residue_bytes.
+  for (int r = 0; r < nres; ++r) {
+    const int ne = res_off[r + 1] - res_off[r];
+    if (rmsd_perres_residue_bytes(ne, 2 * ne + 64) <= PERRES_RESIDUE_MAX) continue;
+    int lo = INT32_MAX, hi = -1;
+    for (int k = res_off[r]; k < res_off[r + 1]; ++k) {
+      lo = std::min(lo, tgt_atoms[k]);
+      hi = std::max(hi, tgt_atoms[k] + 1);
     }
-    if (hi < 0) lo = hi = 0;  // residues without atoms
-    pieces.push_back(span_form ? make_int4(r, r1, lo, hi) : make_int4(r, r1, -1, -1));
+    const int span = hi - lo <= 2 * ne + 64 ? hi - lo : ne;
+    if (rmsd_perres_residue_bytes(ne, span) > PERRES_RESIDUE_MAX)
+      return fail(ctx, RMSD_ERR_ARG, "residue " + std::to_string(r) + " has too many atoms (" +
+                                         std::to_string(ne) + ") for per-residue RMSD");
+  }
+  // Pieces: runs of whole residues.
+  std::vector<int4> pieces;
+  for (int r = 0; r < nres;) {
+    int r1 = r + 1;
+    while (r1 < nres && r1 - r < (center ? PERRES_RES_CENTER : PERRES_RES_PIECE) &&
+           res_off[r1 + 1] - res_off[r] <= PERRES_ENTRIES)
+      ++r1;
+    pieces.push_back(make_int4(r, r1, res_off[r], res_off[r1]));
     r = r1;
   }
-  // Frames per batch: enough (frame, residue) items for the workgroup's lanes,
-  // within PERRES_LDS_BATCH (one frame always runs).
-  int maxnr = 1;
-  for (const int4& p : pieces) maxnr = std::max(maxnr, p.y - p.x);
-  int nfb = std::max(1, PERRES_THREADS / maxnr);
-  auto lds_for = [&](int nf) {
-    size_t m = 0;
-    for (const int4& p : pieces)
-      m = std::max(m, rmsd_perres_lds_bytes(p.y - p.x, res_off[p.y] - res_off[p.x],
-                                            p.z < 0 ? res_off[p.y] - res_off[p.x] : p.w - p.z, nf));
-    return m;
-  };
   if (pieces.size() > 65535) return fail(ctx, RMSD_ERR_ARG, "residue table too large");
-  while (nfb > 1 && lds_for(nfb) > PERRES_LDS_BATCH) --nfb;
-  const size_t lds = lds_for(nfb);
   // Table blob (16-byte aligned sections).
   const size_t o_off = 0;
   const size_t o_tgt = round_up(o_off + sizeof(int32_t) * (nres + 1), 16);
@@ -957,12 +935,11 @@ int rmsd_perres_nofit(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frame
   a.tvec = modify != RMSD_MODIFY_NONE ? tvec : nullptr;
   a.modify = modify == RMSD_MODIFY_ROT_TRANS ? 1 : (modify == RMSD_MODIFY_TRANS ? 2 : 0);
   a.pieces = (const int4*)(dtab + o_pc);
-  a.nfb = nfb;
   a.out = out;
   ctx->marks = 0;
   mark(ctx, 0);
   mark(ctx, 1);
-  HIP_TRY(ctx, rmsd_launch_perres(a, (int)pieces.size(), lds, ctx->stream));
+  HIP_TRY(ctx, rmsd_launch_perres(a, (int)pieces.size(), ctx->stream));
   mark(ctx, 2);
   mark(ctx, 3);
   return RMSD_OK;

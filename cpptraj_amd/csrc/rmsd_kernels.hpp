@@ -318,9 +318,9 @@ struct ApplyArgs {
 
 // Per-residue no-fit RMSD (k_perres.hip).  Residue r owns entries
 // res_off[r] .. res_off[r+1] of tgt_atoms / ref_atoms / tmass / rmass.  pieces:
-// {first residue, end residue, lowest target atom, highest target atom + 1},
-// or {first, end, -1, -1} for a piece that gathers its own atoms; a workgroup
-// stages `nfb` frames' atoms at a time.
+// {first residue, end residue, first entry, end entry}, up to PERRES_ENTRIES
+// entries and PERRES_RES_PIECE (PERRES_RES_CENTER) residues, or one larger
+// residue.
 struct PerresArgs {
   const float* xyz;
   int64_t stride, ld;
@@ -339,16 +339,17 @@ struct PerresArgs {
   const double* tvec;     // 6 per frame (modify 1, 2)
   int modify;             // 0: frames as stored; 1: x' = U (x + t) + r; 2: x + (t + r)
   const int4* pieces;
-  int nfb;
   double* out;            // out[f * nres + r]
 };
-constexpr int PERRES_THREADS = 64;
-constexpr int PERRES_RES_PIECE = 16;                   // residues per piece
-constexpr size_t PERRES_LDS_PIECE = size_t(12) << 10;   // piece budget (LDS bytes at nfb = 1)
-constexpr size_t PERRES_LDS_BATCH = size_t(24) << 10;  // budget when batching frames
-constexpr size_t PERRES_LDS_MAX = size_t(160) << 10;   // one oversized residue alone
-size_t rmsd_perres_lds_bytes(int nres_piece, int nentries, int span, int nfb);
-hipError_t rmsd_launch_perres(const PerresArgs& a, int npieces, size_t lds_bytes, hipStream_t s);
+constexpr int PERRES_THREADS = 256;
+constexpr int PERRES_ENTRIES = 256;   // atoms of a piece
+constexpr int PERRES_RES_PIECE = 128;  // residues of a piece
+constexpr int PERRES_RES_CENTER = 64;  // ... when centred: with their centres in LDS 5
+                                       // workgroups to a CU (320 us) instead of 4 (368)
+// The largest residue accepted: this many bytes by rmsd_perres_residue_bytes.
+constexpr size_t PERRES_RESIDUE_MAX = size_t(160) << 10;
+size_t rmsd_perres_residue_bytes(int natoms, int span);
+hipError_t rmsd_launch_perres(const PerresArgs& a, int npieces, hipStream_t s);
 
 // RMS average correlation (k_avgcorr.hip): one wavefront per window size.
 struct AvgCorrArgs {

@@ -175,3 +175,34 @@ def test_perres_argument_errors(ctx):
     # no frames / no residues: nothing to do
     assert ca.rmsd_perres(X[:0], off, np.arange(6, dtype=np.int32), ref_frames=X,
                           ctx=ctx).shape == (0, 2)
+
+
+@pytest.mark.parametrize("center", [False, True])
+@pytest.mark.parametrize("soa", [False, True])
+@pytest.mark.parametrize("F", [1, 8, 17])
+def test_perres_piece_edges(ctx, oracle, center, soa, F):
+    # Pieces of exactly 256 atoms and of 128 residues, a residue of 256, 257 and
+    # 513 atoms (one to three stretches), residues without atoms between and at
+    # the end; a frame more and a frame less than a batch.
+    import torch
+
+    import cpptraj_amd as ca
+    sizes = [100, 156, 1, 256, 257, 3, 513] + [1] * 140 + [255, 2]
+    rng, X, ref, off, atoms, m = _case(31, F, 1710, sizes, scattered=0)
+    off = np.concatenate([off[:3], off[2:], off[-1:]]).astype(np.int32)
+    U = synth.rotations(rng, F).reshape(F, 3, 3)
+    tv = rng.uniform(-15, 15, size=(F, 6))
+    exp = oracle.perres(X, ref, off, atoms, tmass=m[atoms], use_mass=True, center=center, U=U,
+                        tvec=tv, modify=1)
+    n = X.shape[1] // 3
+
+    def planes(x):
+        x = x.reshape(-1, n, 3)
+        return torch.as_tensor(np.ascontiguousarray(x.transpose(0, 2, 1) if soa else x)).cuda()
+
+    got = ca.rmsd_perres(planes(X) if soa else planes(X).reshape(F, -1), off, atoms,
+                         ref_frames=planes(ref) if soa else planes(ref).reshape(1, -1),
+                         tmass=m[atoms], use_mass=True, center=center, modify="rottrans",
+                         U=torch.as_tensor(U).cuda(), tvec=torch.as_tensor(tv).cuda(), soa=soa,
+                         natom=n if soa else None, ctx=ctx).cpu().numpy()
+    assert np.abs(got - exp).max() <= TOL
