@@ -576,20 +576,38 @@ __global__ __launch_bounds__(SYM_THREADS) void k_symm_final_nofit(SymmArgs a) {
   if (lane == 0) a.rmsd[f] = W < RMSD_SMALL ? -1.0 : (acc < 0.0 ? 0.0 : sqrt(acc / W));
 }
 
-// The per-frame map of every selected atom (SymmetricRmsdCalc::AMap).
-// Grid: x over frames (AMAP_FRAMES per block), y over atoms (256 per block).
+// The per-frame map of every selected atom (SymmetricRmsdCalc::AMap): 4 bytes
+// written per atom and frame, against the store rate.  A thread keeps the group
+// positions of four atoms for AMAP_FRAMES frames and stores them as one dword-
+// aligned 16-byte access: 50,000 frames x 2,000 atoms 193 -> 127 us (400 MB; one
+// atom per thread before).  Grid: x over frames, y over atoms (1024 per block).
 constexpr int AMAP_FRAMES = 8;
+typedef int i32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 __global__ __launch_bounds__(256) void k_symm_amap(SymmArgs a) {
   const int n = a.fs.nsel;
-  const int i = blockIdx.y * 256 + threadIdx.x;
+  const int i = 4 * (blockIdx.y * 256 + threadIdx.x);
   if (i >= n) return;
-  const int p = a.pos[i];
+  const bool quad = i + 4 <= n;
+  int p[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) p[c] = i + c < n ? a.pos[i + c] : -1;
   const int64_t f0 = (int64_t)blockIdx.x * AMAP_FRAMES;
 #pragma unroll
   for (int k = 0; k < AMAP_FRAMES; ++k) {
     const int64_t f = f0 + k;
     if (f >= a.fs.nframes) break;
-    a.amap[f * n + i] = p >= 0 ? a.gmap[f * a.ngatoms + p] : i;
+    const int* gm = a.gmap + f * a.ngatoms;
+    int* out = a.amap + f * n + i;
+    i32x4_a4 v;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) v[c] = p[c] >= 0 ? gm[p[c]] : i + c;
+    if (quad) {
+      *reinterpret_cast<i32x4_a4*>(out) = v;
+    } else {
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        if (i + c < n) out[c] = v[c];
+    }
   }
 }
 
@@ -625,7 +643,7 @@ hipError_t rmsd_launch_symm(const SymmArgs& a, hipStream_t s) {
     hipLaunchKernelGGL((k_symm_final_nofit<false>), grid, block, 0, s, a);
   if (a.amap) {
     const int64_t gx = (F + AMAP_FRAMES - 1) / AMAP_FRAMES;
-    const int gy = (a.fs.nsel + 255) / 256;
+    const int gy = (a.fs.nsel + 1023) / 1024;
     if (gy > 65535) return hipErrorInvalidValue;
     const dim3 g((unsigned)gx, (unsigned)gy);
     hipLaunchKernelGGL(k_symm_amap, g, dim3(256), 0, s, a);

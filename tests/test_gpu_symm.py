@@ -155,6 +155,26 @@ def test_symm_20000_frames(ctx, oracle):
     assert rm.cpu().numpy()[0] < 1e-6
 
 
+@pytest.mark.parametrize("F,natom", [(2, 61), (13, 62), (16, 63), (33, 1025), (9, 1028)])
+def test_symm_map_rows(ctx, oracle, F, natom):
+    # Map rows with 1, 2, 3 and 0 atoms past a multiple of 4, and just past one
+    # block of 1,024; a last block of frames part filled.
+    import torch
+
+    import cpptraj_amd as ca
+    X, ref, groups, m, _ = synth.symm_case(74, F, natom, ngroups=9, compact=True)
+    Xd = torch.as_tensor(X).cuda()
+    R = torch.as_tensor(ref.reshape(1, -1).astype(np.float32)).cuda()
+    md = torch.as_tensor(m).cuda()
+    rm, amap, U, _ = ca.rmsd_symm(Xd, groups, ref_frames=R, mass=md, use_mass=True, want_map=True,
+                                  want_xform=True, ctx=ctx)
+    eo, ao, Uo, _, _ = _oracle(oracle, X, ref.astype(np.float32).astype(np.float64), groups, m,
+                               True, True)
+    assert np.array_equal(amap.cpu().numpy(), ao)
+    assert np.abs(rm.cpu().numpy() - eo).max() <= 1e-9
+    assert np.abs(U.cpu().numpy().reshape(-1, 9) - Uo).max() <= 1e-9
+
+
 def test_symm_no_groups_is_the_fit(ctx):
     import torch
 
