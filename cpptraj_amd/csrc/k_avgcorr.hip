@@ -217,19 +217,19 @@ hipError_t rmsd_launch_avgcorr(const AvgCorrArgs& a, bool first, hipStream_t s) 
 // With the selected coordinates x_f and their per-coordinate mean mu, the
 // prefix sums P_i = sum_{f < i} (x_f - mu) (i = 0..F, P_0 = 0) give the
 // window-w average ending at frame t (i = t + 1, j = i - w) as
-// a = (P_i - P_j) / w + mu.  With d = P_i - P_j, v = mu - mu_c (mu_c the
-// weighted centroid of mu) and the fit centroid c = (sum m d) / (w W) + mu_c:
-//   sum m a y^T       = (Q_i - Q_j) / w + sum m mu y^T
+// a = (P_i - P_j) / w + mu.  The rows lose their centroids, P~_i = P_i - C_i / W
+// with C_i = sum m P_i, so that where molecules diffuse or jump no common
+// translation has to cancel later.  With d = P~_i - P~_j, v = mu - mu_c (mu_c
+// the weighted centroid of mu) and the fit centroid c:
+//   sum m (a - c) y^T = (Q_i - Q_j) / w + sum m v y^T
 //   sum m |a - c|^2   = sum m |d|^2 / w^2 + 2 (L_i - L_j) / w + sum m |v|^2
-//                       - W |(C_i - C_j) / (w W)|^2
-// with per-prefix moments C_i = sum m P_i, Q_i = sum m P_i y^T and
-// L_i = sum m v . P_i.  Only sum m |d|^2 needs all coordinates of a pair:
-// it is a squared distance between two prefix rows, computed from the
-// difference itself (no |P_i|^2 + |P_j|^2 - 2 P_i . P_j cancellation), in
+// with per-prefix moments Q_i = sum m P~_i y^T and L_i = sum m v . P~_i ('first'
+// keeps P_i and C_i: its references move too).  Only sum m |d|^2 needs all
+// coordinates of a pair: it is a squared distance between two prefix rows, in
 // 64 x 64 tiles of (i, j) pairs.  Each tile fits the pairs whose i - j is a
-// window size and sums their RMSDs per diagonal; a last pass adds the
-// per-tile sums of every window in a fixed order.  Subtracting mu first
-// keeps the prefix sums, and the digits their differences lose, small.
+// window size and sums their RMSDs per diagonal; a last pass adds the per-tile
+// sums of every window in a fixed order.  Subtracting mu first keeps the prefix
+// sums, and the digits their differences lose, small.
 namespace {
 
 constexpr int AC_CHUNK = 128;  // frames per scan chunk
@@ -289,7 +289,7 @@ __global__ __launch_bounds__(AC_THREADS) void k_ac_prefix(AvgPrefixArgs a) {
   }
 }
 
-// Constants (row F + 1 of rows): sum m mu (3), sum m mu y^T (9),
+// Constants (row F + 1 of rows): sum m mu (3), sum m v y^T (9),
 // sum m |v|^2 (1).  One wave.
 __global__ __launch_bounds__(64) void k_ac_consts(AvgPrefixArgs a) {
   const int n = a.fs.nsel;
@@ -312,8 +312,8 @@ __global__ __launch_bounds__(64) void k_ac_consts(AvgPrefixArgs a) {
     const double y0 = a.ref ? a.ref[kk] : 0.0, y1 = a.ref ? a.ref[a.ldr + kk] : 0.0,
                  y2 = a.ref ? a.ref[2 * a.ldr + kk] : 0.0;
     for (int c = 0; c < 3; ++c) {
-      const double mm = m * a.mu[3 * kk + c];
       const double vc = a.mu[3 * kk + c] - mc[c];
+      const double mm = m * vc;
       v[3 + 3 * c] += mm * y0;
       v[4 + 3 * c] += mm * y1;
       v[5 + 3 * c] += mm * y2;
@@ -329,7 +329,9 @@ __global__ __launch_bounds__(64) void k_ac_consts(AvgPrefixArgs a) {
   }
 }
 
-// Per prefix row i (0..F): C_i (3), Q_i (9), L_i (1).  One wave per row.
+// Per prefix row i (0..F): C_i (3), Q_i (9), L_i (1).  One wave per row.  With a
+// fixed reference the row loses its centroid first: P~_i = P_i - C_i / W (44 us at
+// 10,000 x 300, the rows written once more; 19 without).
 __global__ __launch_bounds__(64) void k_ac_rows(AvgPrefixArgs a) {
   const int64_t i = blockIdx.x;
   const int n = a.fs.nsel;
@@ -337,7 +339,18 @@ __global__ __launch_bounds__(64) void k_ac_rows(AvgPrefixArgs a) {
   const double* cr = a.rows + (a.fs.nframes + 1) * 13;
   double mc[3];
   for (int c = 0; c < 3; ++c) mc[c] = W > 0.0 ? cr[c] / W : 0.0;
-  const double* Pi = a.P + i * a.k;
+  double* Pi = a.P + i * a.k;
+  double t[3] = {0.0, 0.0, 0.0};
+  if (a.ref) {
+    for (int kk = threadIdx.x; kk < n; kk += 64) {
+      const double sw = a.mass ? sqrt(a.mass[kk]) : 1.0;
+      for (int c = 0; c < 3; ++c) t[c] += sw * Pi[3 * kk + c];
+    }
+    for (int c = 0; c < 3; ++c) {
+      t[c] = rmsd_dev::wave_sum(t[c]);
+      t[c] = W > 0.0 ? t[c] / W : 0.0;
+    }
+  }
   double v[13];
 #pragma unroll
   for (int q = 0; q < 13; ++q) v[q] = 0.0;
@@ -346,7 +359,9 @@ __global__ __launch_bounds__(64) void k_ac_rows(AvgPrefixArgs a) {
     const double y0 = a.ref ? a.ref[kk] : 0.0, y1 = a.ref ? a.ref[a.ldr + kk] : 0.0,
                  y2 = a.ref ? a.ref[2 * a.ldr + kk] : 0.0;
     for (int c = 0; c < 3; ++c) {
-      const double mp = sw * Pi[3 * kk + c];  // m P
+      const double p = Pi[3 * kk + c] - sw * t[c];
+      if (a.ref) Pi[3 * kk + c] = p;
+      const double mp = sw * p;  // m P
       v[c] += mp;
       v[3 + 3 * c] += mp * y0;
       v[4 + 3 * c] += mp * y1;
@@ -361,28 +376,21 @@ __global__ __launch_bounds__(64) void k_ac_rows(AvgPrefixArgs a) {
 }
 
 // The fit of one averaged frame from the difference form's pieces: d2 = sum
-// m |P_i - P_j|^2, the row moments ri and rj, the constants row cm and the
-// reference constants K.
+// m |P~_i - P~_j|^2, the row moments ri and rj, the constants
+// row cm and the reference constants K.
 __device__ __forceinline__ double ac_fit(double d2, const double* ri, const double (&rj)[13],
-                                         const double* cm, const double* K, double iW, double w) {
+                                         const double* cm, const double* K, double w) {
   const double W = K[4];
   if (W < RMSD_SMALL) return -1.0;
-  // 1 / w to the last bit or two: the hardware reciprocal, refined twice
+  // 1 / w: the hardware reciprocal, refined twice (2^-53)
   double iw = __builtin_amdgcn_rcp(w);
   iw = fma(iw, fma(-w, iw, 1.0), iw);
   iw = fma(iw, fma(-w, iw, 1.0), iw);
-  double dc[3], c[3];
-#pragma unroll
-  for (int e = 0; e < 3; ++e) {
-    dc[e] = (ri[e] - rj[e]) * (iw * iW);
-    c[e] = dc[e] + cm[e] * iW;
-  }
   double R[9];
 #pragma unroll
-  for (int e = 0; e < 9; ++e) R[e] = (ri[3 + e] - rj[3 + e]) * iw + cm[3 + e] - c[e / 3] * K[e % 3];
-  const double sx = d2 * (iw * iw) + 2.0 * (ri[12] - rj[12]) * iw + cm[12] -
-                    W * (dc[0] * dc[0] + dc[1] * dc[1] + dc[2] * dc[2]);
-  return rmsd_dev::qcp_rmsd_fast(R, 0.5 * (sx + K[3]), iW, 1);
+  for (int e = 0; e < 9; ++e) R[e] = (ri[3 + e] - rj[3 + e]) * iw + cm[3 + e];
+  const double sx = d2 * (iw * iw) + 2.0 * (ri[12] - rj[12]) * iw + cm[12];
+  return rmsd_dev::qcp_rmsd(R, 0.5 * (sx + K[3]), W, 1);
 }
 
 // Sums of a tile's RMSDs rr[64][AC_LD] along its diagonals: thread dd + 63
@@ -462,7 +470,6 @@ __device__ __forceinline__ void ac_direct(const AvgPrefixArgs& a, int ti, int tj
   }
   // Fits of the pairs on window diagonals.
   const double* cm = a.rows + nrow * 13;
-  const double iW = 1.0 / a.consts[4];
   double* rr = sm;
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
@@ -477,7 +484,7 @@ __device__ __forceinline__ void ac_direct(const AvgPrefixArgs& a, int ti, int tj
       const int64_t i = i0 + il, w = i - j;
       double r = 0.0;
       if (w >= 1 && i < nrow && a.wmap[w] >= 0)
-        r = ac_fit(acc[p][q], a.rows + i * 13, rj, cm, a.consts, iW, (double)w);
+        r = ac_fit(acc[p][q], a.rows + i * 13, rj, cm, a.consts, (double)w);
       rr[il * AC_LD + jl] = r;
     }
   }
@@ -490,26 +497,27 @@ __device__ __forceinline__ void ac_direct(const AvgPrefixArgs& a, int ti, int tj
 // and pair instead of a difference and a multiply-add.  Rows are taken about the
 // middle row m of the column tile, q_i = P_i - P_m, p_j = P_j - P_m:
 //   |P_i - P_j|^2 = |q_i|^2 + |p_j|^2 - 2 q_i . p_j.
-// p_j reaches over at most 32 frames and q_i over about w of them, so what the
-// sum cancels is of the size of the distance itself; where a trajectory makes
-// |P_i - P_j| small against |p_j|, the rounding left, eps |p_j|^2 / w^2 with
-// |p_j| <= 32 frames' deviation and w >= 65, is below eps times the sum
-// m |mu - mu_c|^2 that the fit adds to it.  Nearer the diagonal that does not
-// hold, hence ac_direct there.
+// With |q_i| <= |P_i - P_j| + |p_j| its rounding is a few eps of |P_i - P_j|^2, as
+// the differences' own, and of |p_j|^2, at most 32 frames' deviations from the
+// mean.  The latter, over w^2, has to stay below the reference's sum w |y|^2,
+// which the fit adds to it and rounds itself: a tile where it does not (returns
+// false, before anything is stored) takes the differences.  Deviations that keep
+// one direction for 32 frames have to reach twice the reference's radius of
+// gyration for that, and only in the tiles of the shortest windows.
 //
 // Each of the four waves owns 32 x 32 pairs, four 16 x 16 blocks; a stage of 32
 // coordinates of the 128 rows goes to LDS shifted, the next stage's loads in
-// flight meanwhile.  Bound by the FP64 matrix
-// rate and, after it, the fits' vector FP64.  Tiles come in bands of eight row
+// flight meanwhile.  Bound by the FP64 matrix rate
+// and, after it, the fits' vector FP64.  Tiles come in bands of eight row
 // tiles, an XCD's workgroups in one run of that order, so that tiles running
 // side by side share rows in its L2.  10,000 frames x 300 atoms, all windows: the
-// whole call 2.43 ms against 4.80 with every tile's distances from the
+// whole call 2.46 ms against 4.80 with every tile's distances from the
 // differences; MFMA pipes 54 % busy and vector issue 27 % at 2.1 GHz, three waves
 // per SIMD (four spill: 3.36 ms).  The tiles near the diagonal run in the same
 // launch: 314 of 12,400, alone on the chip they took 286 us.
 typedef __attribute__((ext_vector_type(4))) double f64x4;
 
-__device__ __forceinline__ void ac_gram(const AvgPrefixArgs& a, int ti, int tj, double* sm,
+__device__ __forceinline__ bool ac_gram(const AvgPrefixArgs& a, int ti, int tj, double* sm,
                                         double (*norm)[2 * AC_TILE]) {
   double* si = sm;
   double* sj = sm + AC_KC * AC_LD;
@@ -583,8 +591,10 @@ __device__ __forceinline__ void ac_gram(const AvgPrefixArgs& a, int ti, int tj, 
   }
   norm[t >> 7][t & 127] = sq;
   __syncthreads();  // and the last stage's reads: sm becomes the RMSD tile
+  const double far = norm[0][AC_TILE + lane] + norm[1][AC_TILE + lane];  // |p_j|^2, j0 + lane
+  const double wmin = (double)(AC_TILE * (ti - tj) - (AC_TILE - 1));
+  if (!__all(far <= wmin * wmin * a.consts[3])) return false;  // the same in every wave
   const double* cm = a.rows + nrow * 13;
-  const double iW = 1.0 / a.consts[4];
   // The accumulators hold row lane / 16 + 4 v, column lane % 16, in item v.
 #pragma unroll 1
   for (int q = 0; q < 2; ++q) {
@@ -604,13 +614,14 @@ __device__ __forceinline__ void ac_gram(const AvgPrefixArgs& a, int ti, int tj, 
         if (i < nrow && a.wmap[w] >= 0) {
           const double g = q == 0 ? acc[p][0][v] : acc[p][1][v];
           const double d2 = fmax(norm[0][il] + norm[1][il] + nj - 2.0 * g, 0.0);
-          r = ac_fit(d2, a.rows + i * 13, rj, cm, a.consts, iW, (double)w);
+          r = ac_fit(d2, a.rows + i * 13, rj, cm, a.consts, (double)w);
         }
         sm[il * AC_LD + jl] = r;
       }
   }
   __syncthreads();
   ac_diagonals(a, sm, ti, tj);
+  return true;
 }
 
 // The tiles near the diagonal first: they take longest.
@@ -619,16 +630,16 @@ __global__ __launch_bounds__(AC_THREADS) __attribute__((amdgpu_waves_per_eu(3)))
   __shared__ double sm[AC_LDS];
   __shared__ double norm[2][2 * AC_TILE];
   const int near = a.ntiles - a.ngram;
-  if ((int)blockIdx.x < near) {
-    const int2 tile = a.tiles[blockIdx.x];
-    ac_direct(a, tile.x, tile.y, sm);
-    return;
+  int k = (int)blockIdx.x;
+  if (k >= near) {
+    const int b = k - near;
+    const int w = (b % AC_XCDS) * a.gram_per_xcd + b / AC_XCDS;
+    if (w >= a.ngram) return;  // the whole workgroup
+    k = near + w;
   }
-  const int b = (int)blockIdx.x - near;
-  const int w = (b % AC_XCDS) * a.gram_per_xcd + b / AC_XCDS;
-  if (w >= a.ngram) return;  // the whole workgroup
-  const int2 tile = a.tiles[near + w];
-  ac_gram(a, tile.x, tile.y, sm, norm);
+  const int2 tile = a.tiles[k];
+  if (k >= near && ac_gram(a, tile.x, tile.y, sm, norm)) return;
+  ac_direct(a, tile.x, tile.y, sm);
 }
 
 // Mean and standard deviation per window from the per-tile sums, in a fixed

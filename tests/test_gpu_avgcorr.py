@@ -220,3 +220,63 @@ def test_avgcorr_gram_tile_edges(ctx, F, n, use_mass, offset):
     # SD = sqrt(mean(r^2) - mean(r)^2): rounding of the two means, ~1e-15 r^2,
     # under the root.
     assert float((sd ** 2 - sd2 ** 2)[far].abs().max()) <= 1e-12 * float(ct2.max()) ** 2
+
+
+def _exact_means(X, ref, windows):
+    """Mean RMSD per window in extended precision, and 64 eps E0 / (W r) (64
+    roundings of E0 in the FP64 solve) averaged over each window's fits."""
+    L = np.longdouble
+    F, n = X.shape[:2]
+    X = X.astype(L)
+    P = np.concatenate([np.zeros((1, n, 3), L), np.cumsum(X, 0)])
+    y = ref.astype(L) - ref.astype(L).mean(0)
+    gy = (y * y).sum()
+    mean, tol = [], []
+    for w in windows:
+        a = (P[w:] - P[:-w]) / w
+        a = a - a.mean(1, keepdims=True)
+        S = np.stack([(a[:, :, c, None] * y[None]).sum(1) for c in range(3)], 1)
+        C = np.stack([np.cross(S[:, 1], S[:, 2]), np.cross(S[:, 2], S[:, 0]), np.cross(S[:, 0], S[:, 1])], 1)
+        T = (S * S).sum((1, 2))
+        c2, c1, c0 = -2 * T, -8 * (S[:, 0] * C[:, 0]).sum(1), T * T - 4 * (C * C).sum((1, 2))
+        E0 = ((a * a).sum((1, 2)) + gy) / 2
+        lam = E0.copy()
+        for _ in range(60):
+            lam = lam - (((lam * lam + c2) * lam + c1) * lam + c0) / (4 * lam ** 3 + 2 * c2 * lam + c1)
+        r = np.sqrt(2 * (E0 - lam) / n)
+        mean.append(r.mean())
+        tol.append((64 * np.finfo(float).eps * E0 / (n * r)).mean())
+    return np.array(mean, float), np.array(tol, float)
+
+
+@pytest.mark.parametrize("motion", ["none", "diffusing", "jumping", "breathing 3", "breathing 10"])
+def test_avgcorr_large_motions(ctx, motion):
+    """Trajectories whose prefix sums are large against their differences: common
+    translations of 8,192 A, and internal motion of up to ten times the
+    reference's size with a period of 65 frames (10: tiles that leave the product
+    for the differences).  Coordinates are multiples of 2^-10 A, 256 frames and
+    16 atoms: prefix sums, means and centroids are exact in FP64, what is left is
+    the solve's rounding."""
+    import torch
+
+    import cpptraj_amd as ca
+    F, n = 256, 16
+    rng = np.random.default_rng(17)
+    u = rng.normal(size=(n, 3))
+    chain = np.cumsum(3.8 * u / np.linalg.norm(u, axis=1)[:, None], 0)
+    chain -= chain.mean(0)
+    X = chain + rng.normal(scale=0.5, size=(F, n, 3))
+    f = np.arange(F)[:, None, None]
+    if motion == "diffusing":
+        X += np.cumsum(np.round(rng.normal(scale=50.0, size=(F, 1, 3))), 0)
+    elif motion == "jumping":
+        X += np.where(f % 65 < 32, 8192.0, -8192.0)
+    elif motion != "none":
+        X *= 1 + float(motion.split()[1]) * np.sin(2 * np.pi * f / 65)
+    X = (np.round(X * 1024) / 1024).astype(np.float32)
+    assert np.array_equal(X.astype(np.float64) * 1024, np.round(X.astype(np.float64) * 1024))
+    ref = (np.round((chain + rng.normal(scale=0.3, size=(n, 3))) * 1024) / 1024).astype(np.float32)
+    w, ct, _ = _avgcorr(ca, ctx, torch.as_tensor(X.reshape(F, -1)).cuda(),
+                        ref_frames=torch.as_tensor(ref.reshape(1, -1)).cuda(), method="prefix")
+    exp, tol = _exact_means(X, ref, w)
+    assert np.all(np.abs(ct.cpu().numpy() - exp) <= tol)
