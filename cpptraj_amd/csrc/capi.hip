@@ -204,26 +204,29 @@ FitPlan fit_plan(const rmsd_frames& frames, const rmsd_frames& ref, int ref_fram
 
 int fit_enqueue(rmsd_ctx* c, const FitPlan& plan, const FitBuffers& b, const rmsd_frames& frames,
                 const rmsd_frames& ref, int ref_frame, int use_mass, int modify, double* rmsd,
-                double* U, double* tvec) {
+                double* U, double* tvec, bool timed) {
   const FrameSetDev F = to_dev(frames);
   const FrameSetDev R = to_dev(ref);
   const double* tmass = use_mass ? frames.mass : nullptr;
   const double* rmass = use_mass ? ref.mass : nullptr;
   double* ref_trans = b.ref ? b.ref + 3 * round_up(frames.nsel, 4) : nullptr;
   double* wpad = use_mass ? b.wpad : nullptr;
-  mark(c, 0);
+  auto stage = [&](int k) {
+    if (timed) mark(c, k);
+  };
+  stage(0);
   if (plan.reference())
     HIP_TRY(c, rmsd_launch_ref_prep(R, ref_frame, rmass, tmass, plan.fit ? 1 : 0, b.ref, ref_trans,
                                     b.consts, wpad, c->stream));
-  mark(c, 1);
+  stage(1);
   if (!plan.fit) {
     NofitArgs a;
     a.fs = F;
     a.mass = wpad;
     a.ref = b.ref;
     HIP_TRY(c, rmsd_launch_nofit_frames(a, b.consts, rmsd, c->stream));
-    mark(c, 2);
-    mark(c, 3);
+    stage(2);
+    stage(3);
     return RMSD_OK;
   }
   if (plan.fused) {
@@ -243,8 +246,8 @@ int fit_enqueue(rmsd_ctx* c, const FitPlan& plan, const FitBuffers& b, const rms
     a.U = U;
     a.tvec = tvec;
     HIP_TRY(c, rmsd_launch_fit_fused(a, c->stream));
-    mark(c, 2);
-    mark(c, 3);
+    stage(2);
+    stage(3);
     return RMSD_OK;
   }
   FitArgs fa;
@@ -254,7 +257,7 @@ int fit_enqueue(rmsd_ctx* c, const FitPlan& plan, const FitBuffers& b, const rms
   fa.consts = b.consts;
   fa.moments = b.moments;
   HIP_TRY(c, rmsd_launch_fit_moments(fa, c->stream));
-  mark(c, 2);
+  stage(2);
   SolveArgs sa;
   sa.moments = b.moments;
   sa.consts = b.consts;
@@ -277,7 +280,7 @@ int fit_enqueue(rmsd_ctx* c, const FitPlan& plan, const FitBuffers& b, const rms
     ap.xform = b.xform;
     HIP_TRY(c, rmsd_launch_apply(ap, modify == RMSD_MODIFY_ROT_TRANS ? 1 : 2, c->stream));
   }
-  mark(c, 3);
+  stage(3);
   return RMSD_OK;
 }
 
@@ -714,7 +717,8 @@ int rmsd_fit_to_ref(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frames*
     if (!b.xform) return st;
   }
   ctx->marks = 0;
-  return fit_enqueue(ctx, plan, b, *frames, *ref, ref_frame, use_mass, modify, rmsd, U, tvec);
+  return fit_enqueue(ctx, plan, b, *frames, *ref, ref_frame, use_mass, modify, rmsd, U, tvec,
+                     true);
 }
 
 int rmsd_fit_pairs(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frames* refs, int fit,

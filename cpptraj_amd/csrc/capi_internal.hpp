@@ -93,7 +93,8 @@ void* scratch(rmsd_ctx* c, const char* name, size_t bytes, int* status);
 int check_frames(rmsd_ctx* c, const rmsd_frames* f, const char* what);
 FrameSetDev to_dev(const rmsd_frames& f);
 // The fit of rmsd_fit_to_ref in two steps (capi.hip): which kernels a checked
-// call takes, and so which buffers, then the launches on the context's stream.
+// call takes, and so which buffers, then the launches on the context's stream
+// (timed: with the stage marks of a profiled call).
 struct FitPlan {
   bool fit = false, fused = false, inref = false;
   bool reference() const { return !inref; }              // ref, consts (and wpad with masses)
@@ -111,7 +112,7 @@ FitPlan fit_plan(const rmsd_frames& frames, const rmsd_frames& ref, int ref_fram
                  int modify);
 int fit_enqueue(rmsd_ctx* c, const FitPlan& plan, const FitBuffers& b, const rmsd_frames& frames,
                 const rmsd_frames& ref, int ref_frame, int use_mass, int modify, double* rmsd,
-                double* U, double* tvec);
+                double* U, double* tvec, bool timed);
 std::vector<int2> grouped_tiles(int nbr, int nbc, int tri, int tr = TILE, int tc = TILE);
 int64_t round_up(int64_t x, int64_t m);
 // Coefficients of the per-pair error bound for a precision and chunk count.

@@ -126,7 +126,9 @@ int rmsd_fit_to_ref_noalloc(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd
   }
   if (plan.moments()) b.moments = base + lay.moments;
   if (plan.xform(modify)) b.xform = base + lay.xform;
-  return fit_enqueue(ctx, plan, b, *frames, *ref, ref_frame, use_mass, modify, rmsd, U, tvec);
+  // No stage marks: the context's events must not become part of a capture.
+  return fit_enqueue(ctx, plan, b, *frames, *ref, ref_frame, use_mass, modify, rmsd, U, tvec,
+                     false);
 }
 
 }  // extern "C"

@@ -77,3 +77,41 @@ def test_noalloc_rejects_calls_beyond_its_scratch(ctx):
                                    0, C.c_void_p(out.data_ptr()), None, None)
     assert rc == 1
     assert "RMSD_NOALLOC_SCRATCH_BYTES" in ctx._L.rmsd_last_error(ctx.handle).decode()
+
+
+def test_noalloc_leaves_the_stage_times_alone():
+    """Stage times belong to the last rmsd_fit_to_ref: the allocation-free call
+    records no events, so that it can be captured with profiling on.  The
+    captured call's replays give the eager call's bits."""
+    import torch
+    import cpptraj_amd as ca
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        ctx = ca.Context(0)
+        L = _bind(ctx._L)
+        X = torch.as_tensor(synth.noisy(5, 900, 200, 0.7)).cuda()
+        R = X[:1].clone()
+        d, r = ca.frames_desc(X), ca.frames_desc(R)
+        out, got = (torch.zeros(900, dtype=torch.float64, device="cuda") for _ in range(2))
+
+        def call(fn, to):
+            ctx.check(fn(ctx.handle, C.byref(d), C.byref(r), 0, 1, 0, 0,
+                         C.c_void_p(to.data_ptr()), None, None))
+
+        ctx.set_profiling(True)
+        call(L.rmsd_fit_to_ref, out)
+        times = ctx.stage_ms()
+        call(L.rmsd_fit_to_ref_noalloc, got)
+        stream.synchronize()
+        assert ctx.stage_ms() == times
+        assert torch.equal(got, out)
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=stream):
+            call(L.rmsd_fit_to_ref_noalloc, got)
+        assert ctx.stage_ms() == times
+        for _ in range(3):
+            got.zero_()
+            g.replay()
+            stream.synchronize()
+            assert torch.equal(got, out)
+        ctx.set_profiling(False)
