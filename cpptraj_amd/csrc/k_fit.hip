@@ -715,8 +715,7 @@ hipError_t rmsd_launch_fit_moments(const FitArgs& a, hipStream_t s) {
   if (nf == 0) return hipSuccess;
   const bool vec = a.fs.sel == nullptr && a.fs.ld > 0 && (a.fs.ld % 4) == 0 &&
                    (a.fs.stride % 4) == 0 && ((uintptr_t)a.fs.xyz % 16) == 0;
-  // Quads of atoms, unless they would leave half of a wave's lanes idle.
-  const bool quads = a.fs.sel == nullptr && a.fs.nsel > FIT_SINGLE_ATOMS;
+  const bool quads = a.fs.sel == nullptr && !rmsd_fit_single(a.fs.nsel, a.fs.ld > 0, false);
   const bool aos4 = quads && a.fs.ld == 0, soa = quads && a.fs.ld > 0;
   const bool w = a.mass != nullptr;
   // Wave-per-frame path whenever the reference fits in LDS (up to 5120

@@ -362,9 +362,11 @@ hipError_t launch(const FitFusedArgs& a, int ldr, hipStream_t s) {
 
 template <int OP>
 hipError_t launch_held(const FitFusedArgs& a, int held, int ldr, hipStream_t s) {
+  // As the moment kernels where those take the longer calls.
+  const bool single = rmsd_fit_single(held, a.fs.ld > 0, OP != OP_FIT || a.mode != 0);
   if (a.ref == nullptr) {
     if (held <= 64) return launch<OP, 64, 1, 1, 1, true>(a, ldr, s);
-    if (held <= FIT_SINGLE_ATOMS) return launch<OP, 64, 1, 2, 1, true>(a, ldr, s);
+    if (single) return launch<OP, 64, 1, 2, 1, true>(a, ldr, s);
     if (held <= 256) return launch<OP, 64, 1, 1, 4, true>(a, ldr, s);
     if (held <= 512) return launch<OP, 64, 1, 2, 4, true>(a, ldr, s);
     return launch<OP, 64, 1, 4, 4, true>(a, ldr, s);
@@ -372,7 +374,7 @@ hipError_t launch_held(const FitFusedArgs& a, int held, int ldr, hipStream_t s) 
   const bool many = a.fs.nframes >= FIT_MANY_FRAMES;
   if (held <= 64)
     return many ? launch<OP, 64, 8, 1, 1>(a, ldr, s) : launch<OP, 64, 1, 1, 1>(a, ldr, s);
-  if (held <= FIT_SINGLE_ATOMS)
+  if (single)
     return many ? launch<OP, 64, 4, 2, 1>(a, ldr, s) : launch<OP, 64, 1, 2, 1>(a, ldr, s);
   if (held <= 256)
     return many ? launch<OP, 64, 2, 1, 4>(a, ldr, s) : launch<OP, 64, 1, 1, 4>(a, ldr, s);

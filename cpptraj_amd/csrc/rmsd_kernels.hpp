@@ -270,7 +270,16 @@ struct FitFusedArgs {
   const double* gout = nullptr;  // gradient only: d loss / d RMSD per frame
   void* grad = nullptr;          // [frame][nsel][3], FP64 or FP32
 };
-constexpr int FIT_SINGLE_ATOMS = 128;   // up to here a lane takes single atoms, beyond quads
+// Whether a lane of the fit kernels takes single atoms of a frame of n, not quads
+// (16-byte accesses, but idle lanes).  Where the frame is held for an update or a
+// gradient, up to 128.  Where it is read once, 200,000 frames, single atoms against
+// quads in us: AoS 64 atoms 133 / 145, 68 atoms 151 / 131, 128 atoms 175 / 143; SoA
+// 96 atoms 162 / 162, 101 (a tail of one) 161 / 184, 112 176 / 165, 128 177 / 165.
+inline bool rmsd_fit_single(int n, bool soa, bool held) {
+  if (held) return n <= 128;
+  if (!soa) return n <= 64;
+  return n <= 104 || (n <= 128 && n % 4 != 0);
+}
 constexpr int FIT_MANY_FRAMES = 16384;  // from here a wave takes several small frames
 constexpr int FIT_FUSED_FRAMES = 1024;  // without update: more frames take the moment kernels
 constexpr int FIT_INREF_FRAMES = 512;   // more frames: the reference is prepared once, before

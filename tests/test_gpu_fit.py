@@ -217,7 +217,7 @@ def test_fit_in_registers_edges(oracle, ctx, n, layout, modify):
 
 
 @pytest.mark.parametrize("layout", ["aos", "soa", "sel"])
-@pytest.mark.parametrize("n", [30, 331, 512, 1023])
+@pytest.mark.parametrize("n", [30, 64, 65, 105, 108, 128, 331, 512, 1023])
 def test_fit_same_bits_for_any_frame_count(ctx, n, layout):
     """A frame's results do not depend on how many frames the call has: the
     reference prepared per workgroup, once before, or the moment kernels."""
