@@ -47,9 +47,11 @@ __device__ __forceinline__ float fcoord(const FrameSetDev& fs, int64_t f, int k,
 // workgroup 1 runs it from LDS (masses staged by all its threads) beside the
 // centring in workgroup 0.  One thread summing straight from memory, behind the
 // centring, took 140 us for 2,000 masses and 212 us for 3,000 (a load's latency
-// per few masses); now 13 and 19 us.  Workgroup 0 is
-// alone on the chip and bound by the latency of its trips over the atoms, hence
-// 1,024 threads for more than two trips of 256.
+// per few masses); now 12 and 17 us.  Workgroup 0 is alone on the chip and bound
+// by the latency of its trips over the atoms and by its barriers: 256 / 512 /
+// 1,024 threads 6.5 / 6.3 / 10.6 us at 1,000 unweighted atoms, 9.7 / 8.1 / 11.6 at
+// 2,000, 17.4 / 12.1 / 13.8 at 5,000; with masses, whose staging more threads
+// shorten, 12.3 / 11.6 / 11.9 at 2,000, 18.6 / 17.4 / 16.8 at 3,000.
 constexpr int REF_THREADS = 1024;
 constexpr int REF_STAGE = 2048;  // masses per LDS stage
 
@@ -670,7 +672,7 @@ hipError_t rmsd_launch_ref_prep(const FrameSetDev& fs, int f, const double* rmas
                                 const double* tmass, int center, double* ref_out,
                                 double* ref_trans, double* consts, double* wpad, hipStream_t s) {
   const int ldr = (fs.nsel + 3) & ~3;
-  const int threads = fs.nsel <= 512 ? 256 : REF_THREADS;
+  const int threads = fs.nsel <= 512 ? 256 : tmass && fs.nsel > REF_STAGE ? REF_THREADS : 512;
   hipLaunchKernelGGL(k_ref_prep, dim3(tmass ? 2 : 1), dim3(threads), 0, s, fs, f, rmass, tmass,
                      center, ldr, ref_out, ref_trans, consts, wpad);
   return hipGetLastError();
