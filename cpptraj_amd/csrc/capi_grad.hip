@@ -31,7 +31,7 @@ int fit_backward(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frames* re
   const double* rmass = use_mass ? ref->mass : nullptr;
   // The rotations are recomputed (moments + QCP) rather than kept from the
   // forward call; with the frame held in registers that reads nothing twice.
-  const bool fused = rmsd_fit_grad_fits(F);
+  const bool fused = rmsd_fit_grad_fits(F, f32);
   const bool inref = fused && rmsd_fit_inref_fits(n, n, frames->nframes, 0);
   double* refbuf = nullptr;
   double* ref_trans = nullptr;

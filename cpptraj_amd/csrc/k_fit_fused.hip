@@ -419,14 +419,21 @@ hipError_t rmsd_launch_fit_fused(const FitFusedArgs& a, hipStream_t s) {
 // The gradient holds the fitted atoms as the update holds all of them: the
 // same sizes, and frames without a selection.  4,096 x 2,000 weighted, FP32 out:
 // 60 us (3.3 TB/s) in place of moments, solve, gradient in FP64 and a
-// conversion (25 + 5 + 51 + 60).
-bool rmsd_fit_grad_fits(const FrameSetDev& fs) {
-  return !fs.sel && rmsd_fit_fused_fits(fs.nsel, fs.nsel, fs.nframes, 1);
+// conversion (25 + 5 + 51 + 60).  FP64 out, its 24 bytes per atom written in
+// strided pieces, only up to FIT_GRAD64_ATOMS atoms in all frames where lanes take
+// quads: beyond, the separate kernels store full lines and read the frames from
+// the caches a second time.  This form against those, us: 700 x 3,000 40 / 49,
+// 6,000 x 300 36 / 38, 1,500 x 1,500 44 / 42, 3,000 x 800 47 / 43, 6,000 x 1,500
+// 123 / 90; single atoms 40,000 x 128 64 / 73.
+bool rmsd_fit_grad_fits(const FrameSetDev& fs, bool f32) {
+  if (fs.sel || !rmsd_fit_fused_fits(fs.nsel, fs.nsel, fs.nframes, 1)) return false;
+  return f32 || rmsd_fit_single(fs.nsel, fs.ld > 0, true) ||
+         (int64_t)fs.nframes * fs.nsel <= FIT_GRAD64_ATOMS;
 }
 
 hipError_t rmsd_launch_fit_grad_fused(const FitFusedArgs& a, bool f32, hipStream_t s) {
   if (a.fs.nframes <= 0) return hipSuccess;
-  if (!rmsd_fit_grad_fits(a.fs) || a.mode) return hipErrorInvalidValue;
+  if (!rmsd_fit_grad_fits(a.fs, f32) || a.mode) return hipErrorInvalidValue;
   if (!a.ref && !rmsd_fit_inref_fits(a.fs.nsel, a.fs.nsel, a.fs.nframes, 0))
     return hipErrorInvalidValue;
   const int ldr = (a.fs.nsel + 3) & ~3;

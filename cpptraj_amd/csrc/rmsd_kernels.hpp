@@ -282,12 +282,13 @@ inline bool rmsd_fit_single(int n, bool soa, bool held) {
 }
 constexpr int FIT_MANY_FRAMES = 16384;  // from here a wave takes several small frames
 constexpr int FIT_FUSED_FRAMES = 1024;  // without update: more frames take the moment kernels
+constexpr int64_t FIT_GRAD64_ATOMS = 9 << 18;  // FP64 gradient: atoms of all frames, beyond quads
 constexpr int FIT_INREF_FRAMES = 512;   // more frames: the reference is prepared once, before
 bool rmsd_fit_fused_fits(int natom, int nsel, int nframes, int mode);
 bool rmsd_fit_inref_fits(int natom, int nsel, int nframes, int mode);
 hipError_t rmsd_launch_fit_fused(const FitFusedArgs& a, hipStream_t s);
 // The gradient of the fit (mode 0, no selection; rmsd, U, tvec unused) the same way.
-bool rmsd_fit_grad_fits(const FrameSetDev& fs);
+bool rmsd_fit_grad_fits(const FrameSetDev& fs, bool f32);
 hipError_t rmsd_launch_fit_grad_fused(const FitFusedArgs& a, bool f32, hipStream_t s);
 
 // Fit of target frame f of T to reference frame f of R, every f (k_fit.hip,

@@ -192,3 +192,26 @@ def test_pairwise_backward_edges(oracle, ctx, FA, FB, n, use_mass):
                                            A[q].astype(np.float64), m, use_mass)[1]
     assert np.abs(ga[i].cpu().numpy() - ei).max() <= 1e-9 * np.abs(ei).max()
     assert np.abs(gb[j].cpu().numpy() - ej).max() <= 1e-9 * np.abs(ej).max()
+
+
+@pytest.mark.parametrize("F,n", [(2359, 1000), (2360, 1000), (18431, 128), (18433, 128), (18433, 131)])
+def test_fit_backward_either_side_of_the_fp64_line(ctx, F, n):
+    """FP64 gradients of 9 * 2^18 atoms and more leave the one-launch form (beyond
+    128 atoms a frame): both sides of that line against the selection's kernels."""
+    import ctypes as C
+    import torch
+    import cpptraj_amd as ca
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n)
+    base = torch.randn((1, n, 3), generator=g, device="cuda") * 10
+    X = base + torch.randn((F, n, 3), generator=g, device="cuda")
+    m = dev(synth.masses(np.random.default_rng(n), n))
+    gr = torch.linspace(-1.0, 2.0, F, dtype=torch.float64, device="cuda")
+    out = []
+    for sel in (None, torch.arange(n, dtype=torch.int32, device="cuda")):
+        d, r = ca.frames_desc(X, sel, m), ca.frames_desc(base, sel, m)
+        out.append(torch.full((F, n, 3), 9.0, dtype=torch.float64, device="cuda"))
+        ctx.check(ctx._L.rmsd_fit_backward(ctx.handle, C.byref(d), C.byref(r), 0, 1,
+                                           C.c_void_p(gr.data_ptr()),
+                                           C.c_void_p(out[-1].data_ptr())))
+    assert float((out[0] - out[1]).abs().max()) <= 1e-9 * float(out[1].abs().max())
