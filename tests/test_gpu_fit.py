@@ -251,3 +251,36 @@ def test_fit_reference_among_the_rewritten_frames(oracle, ctx):
     assert_rmsd_close(r.cpu().numpy(), r_o, X)
     ulp = np.spacing(np.abs(fo).astype(np.float32))
     assert np.all(np.abs(Xd.cpu().numpy() - fo) <= 2 * ulp + 1e-30)
+
+
+@pytest.mark.parametrize("modify", ["rottrans", "norotate"])
+@pytest.mark.parametrize("layout", ["aos", "soa", "sel"])
+@pytest.mark.parametrize("n", [50, 64, 66, 128, 131, 200, 255, 256])
+def test_fit_several_frames_per_wave(ctx, n, layout, modify):
+    """From 16,384 frames on a wave takes 8, 4 or 2 small frames (the last group
+    part filled): the bits of the same frames in calls below that."""
+    import cpptraj_amd as ca
+    import torch
+    F = 16384 + 5
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n)
+    X3 = torch.randn((1, n, 3), generator=g, device="cuda") * 10
+    R3 = X3 + torch.randn((1, n, 3), generator=g, device="cuda")
+    X3 = X3 + torch.randn((F, n, 3), generator=g, device="cuda")
+    soa = layout == "soa"
+    sel = torch.arange(0, n, 3, dtype=torch.int32, device="cuda") if layout == "sel" else None
+    um = n % 2 == 0
+    m = dev(synth.masses(np.random.default_rng(n), n if sel is None else sel.numel()))
+
+    def lay(x):
+        return x.permute(0, 2, 1).contiguous() if soa else x.reshape(len(x), -1).clone()
+
+    def fit(x):
+        x = lay(x)
+        out = ca.rmsd_fit(x, lay(R3), mask=sel, mass=m, use_mass=um, modify=modify,
+                          save_matrices=True, save_vectors=True, soa=soa, ctx=ctx)
+        return (*out, x)
+    whole = fit(X3)
+    for s in (slice(0, 9000), slice(9000, F)):
+        for a, b in zip(whole, fit(X3[s])):
+            assert torch.equal(a[s], b)

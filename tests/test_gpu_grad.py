@@ -215,3 +215,36 @@ def test_fit_backward_either_side_of_the_fp64_line(ctx, F, n):
                                            C.c_void_p(gr.data_ptr()),
                                            C.c_void_p(out[-1].data_ptr())))
     assert float((out[0] - out[1]).abs().max()) <= 1e-9 * float(out[1].abs().max())
+
+
+@pytest.mark.parametrize("use_mass", [0, 1])
+@pytest.mark.parametrize("n", [50, 64, 66, 128, 131, 200, 255, 256])
+def test_fit_backward_several_frames_per_wave(ctx, n, use_mass):
+    """From 16,384 frames on a wave takes 8, 4 or 2 small frames: the bits of the
+    same frames in calls below that (FP64 as far as the larger call stays in the
+    one-launch form)."""
+    import ctypes as C
+    import torch
+    import cpptraj_amd as ca
+    F = 16384 + 5
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n)
+    base = torch.randn((1, n, 3), generator=g, device="cuda") * 10
+    X = base + torch.randn((F, n, 3), generator=g, device="cuda")
+    m = dev(synth.masses(np.random.default_rng(n), n))
+    gr = torch.linspace(-1.0, 2.0, F, dtype=torch.float64, device="cuda")
+    for fn, dt in ((ctx._L.rmsd_fit_backward_f32, torch.float32),
+                   (ctx._L.rmsd_fit_backward, torch.float64)):
+        if dt == torch.float64 and n > 131:
+            continue
+
+        def grad(s):
+            x, q = X[s], gr[s]
+            d, r = ca.frames_desc(x, None, m), ca.frames_desc(base, None, m)
+            out = torch.full((len(x), n, 3), 9.0, dtype=dt, device="cuda")
+            ctx.check(fn(ctx.handle, C.byref(d), C.byref(r), 0, use_mass,
+                         C.c_void_p(q.data_ptr()), C.c_void_p(out.data_ptr())))
+            return out
+        whole = grad(slice(0, F))
+        for s in (slice(0, 9000), slice(9000, F)):
+            assert torch.equal(whole[s], grad(s))
