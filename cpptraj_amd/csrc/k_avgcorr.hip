@@ -438,18 +438,41 @@ __device__ __forceinline__ void ac_direct(const AvgPrefixArgs& a, int ti, int tj
   for (int p = 0; p < 4; ++p)
 #pragma unroll
     for (int q = 0; q < 4; ++q) acc[p][q] = 0.0;
-  // Staging: thread t loads coordinate (t % 32) of rows (t / 32) + 8 r.
+  // Staging: thread t takes coordinate (t % 32) of rows (t / 32) + 8 r, the next
+  // stage's in flight meanwhile.  Rows and coordinates past the end are read from
+  // the last row and coordinate 0, so that no load waits behind a branch (with
+  // branches and no prefetch these few tiles' latency bound the small calls: 128 x
+  // 300 332 -> 241 us, 2,000 x 300, every tenth window, 426 -> 336).
   const int lc = t & (AC_KC - 1), lr = t >> 5;
-  for (int k0 = 0; k0 < a.k; k0 += AC_KC) {
-    const int kc = k0 + lc;
+  const auto bi = gp(a.P + i0 * a.k), bj = gp(a.P + j0 * a.k);
+  const int ni = (int)(nrow - i0), nj = (int)(nrow - j0);
+  int oi[8], oj[8];
 #pragma unroll
-    for (int r = 0; r < AC_TILE / 8; ++r) {
-      const int row = lr + 8 * r;
-      const int64_t gi = i0 + row, gj = j0 + row;
-      si[lc * AC_LD + row] = (kc < a.k && gi < nrow) ? a.P[gi * a.k + kc] : 0.0;
-      sj[lc * AC_LD + row] = (kc < a.k && gj < nrow) ? a.P[gj * a.k + kc] : 0.0;
+  for (int r = 0; r < 8; ++r) {
+    const int row = lr + 8 * r;
+    oi[r] = (row < ni ? row : ni - 1) * a.k;
+    oj[r] = (row < nj ? row : nj - 1) * a.k;
+  }
+  double vi[8], vj[8];
+  auto fetch = [&](int k0) {
+    const int kc = k0 + lc < a.k ? k0 + lc : 0;
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      vi[r] = bi[oi[r] + kc];
+      vj[r] = bj[oj[r] + kc];
+    }
+  };
+  fetch(0);
+  for (int k0 = 0; k0 < a.k; k0 += AC_KC) {
+    const bool in = k0 + lc < a.k;
+    __syncthreads();  // the last stage's reads
+#pragma unroll
+    for (int r = 0; r < 8; ++r) {
+      si[lc * AC_LD + lr + 8 * r] = in ? vi[r] : 0.0;
+      sj[lc * AC_LD + lr + 8 * r] = in ? vj[r] : 0.0;
     }
     __syncthreads();
+    if (k0 + AC_KC < a.k) fetch(k0 + AC_KC);
 #pragma unroll 4
     for (int c = 0; c < AC_KC; ++c) {
       double pi[4], pj[4];
@@ -466,8 +489,8 @@ __device__ __forceinline__ void ac_direct(const AvgPrefixArgs& a, int ti, int tj
           acc[p][q] = fma(d, d, acc[p][q]);
         }
     }
-    __syncthreads();
   }
+  __syncthreads();
   // Fits of the pairs on window diagonals.
   const double* cm = a.rows + nrow * 13;
   double* rr = sm;
@@ -511,10 +534,10 @@ __device__ __forceinline__ void ac_direct(const AvgPrefixArgs& a, int ti, int tj
 // and, after it, the fits' vector FP64.  Tiles come in bands of eight row
 // tiles, an XCD's workgroups in one run of that order, so that tiles running
 // side by side share rows in its L2.  10,000 frames x 300 atoms, all windows: the
-// whole call 2.46 ms against 4.80 with every tile's distances from the
+// whole call 2.43 ms against 4.80 with every tile's distances from the
 // differences; MFMA pipes 54 % busy and vector issue 27 % at 2.1 GHz, three waves
 // per SIMD (four spill: 3.36 ms).  The tiles near the diagonal run in the same
-// launch: 314 of 12,400, alone on the chip they took 286 us.
+// launch: 314 of 12,400.
 typedef __attribute__((ext_vector_type(4))) double f64x4;
 
 __device__ __forceinline__ bool ac_gram(const AvgPrefixArgs& a, int ti, int tj, double* sm,
