@@ -324,6 +324,55 @@ struct Packed {
   double* cen = nullptr;  // MFMA forms: per-frame centroids (4 doubles)
 };
 
+// The pieces of k_perres_lane: runs of whole residues that fit PERRES_LANE_PIECE at
+// one frame.  A piece stages its target atom span, or gathers its own atoms when
+// the span is more than twice their number (lo = -1); a residue that would switch
+// a run from one form to the other starts a new piece.  nfb: enough (frame,
+// residue) items for the workgroup's lanes, within PERRES_LANE_BATCH (one frame
+// always runs).
+std::vector<int4> perres_lane_pieces(int nres, const int32_t* res_off, const int32_t* tgt_atoms,
+                                     int* nfb, size_t* lds) {
+  std::vector<int4> pieces;
+  auto staged = [](int span, int ne) { return span <= 2 * ne + 64 ? span : -1; };
+  int maxnr = 1;
+  for (int r = 0; r < nres;) {
+    int lo = INT32_MAX, hi = -1, r1 = r;
+    bool span_form = true;
+    while (r1 < nres && r1 - r < PERRES_LANE_RESIDUES) {
+      int l2 = lo, h2 = hi;
+      for (int k = res_off[r1]; k < res_off[r1 + 1]; ++k) {
+        l2 = std::min(l2, tgt_atoms[k]);
+        h2 = std::max(h2, tgt_atoms[k] + 1);
+      }
+      const int ne = res_off[r1 + 1] - res_off[r];
+      const int span = h2 > l2 ? h2 - l2 : 0;
+      const bool sf = staged(span, ne) >= 0;
+      const size_t b = rmsd_perres_lane_bytes(r1 + 1 - r, ne, sf ? span : ne, 1);
+      if (r1 > r && (b > PERRES_LANE_PIECE || sf != span_form)) break;
+      lo = l2;
+      hi = h2;
+      span_form = sf;
+      ++r1;
+    }
+    if (hi < 0) lo = hi = 0;  // residues without atoms
+    pieces.push_back(span_form ? make_int4(r, r1, lo, hi) : make_int4(r, r1, -1, -1));
+    maxnr = std::max(maxnr, r1 - r);
+    r = r1;
+  }
+  auto lds_for = [&](int nf) {
+    size_t m = 0;
+    for (const int4& p : pieces) {
+      const int ne = res_off[p.y] - res_off[p.x];
+      m = std::max(m, rmsd_perres_lane_bytes(p.y - p.x, ne, p.z < 0 ? ne : p.w - p.z, nf));
+    }
+    return m;
+  };
+  *nfb = std::max(1, PERRES_LANE_THREADS / maxnr);
+  while (*nfb > 1 && lds_for(*nfb) > PERRES_LANE_BATCH) --*nfb;
+  *lds = lds_for(*nfb);
+  return pieces;
+}
+
 int prepare_set(rmsd_ctx* c, const FrameSetDev& fs, const double* cmass, const double* smass,
                 int prec, int Kp, const double* T, const double* gT, double* M, bool sum_weights,
                 const char* tag, Packed* out) {
@@ -892,6 +941,28 @@ int rmsd_perres_nofit(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frame
     r = r1;
   }
   if (pieces.size() > 65535) return fail(ctx, RMSD_ERR_ARG, "residue table too large");
+  int most = 0, lo = INT32_MAX, hi = 0;
+  for (int r = 0; r < nres; ++r) most = std::max(most, res_off[r + 1] - res_off[r]);
+  auto by_lane_for = [&](int span) {
+    return rmsd_perres_by_lane(
+        center != 0, modify == RMSD_MODIFY_ROT_TRANS ? 1 : (modify == RMSD_MODIFY_TRANS ? 2 : 0),
+        (int)pieces.size(), nres, L, most, span);
+  };
+  bool by_lane = by_lane_for(0);
+  if (by_lane && L) {  // the span of the atoms only where it can matter
+    for (int k = 0; k < L; ++k) {
+      lo = std::min(lo, tgt_atoms[k]);
+      hi = std::max(hi, tgt_atoms[k] + 1);
+    }
+    by_lane = by_lane_for(hi - lo);
+  }
+  int nfb = 0;
+  size_t lane_lds = 0;
+  if (by_lane) {
+    std::vector<int4> runs = perres_lane_pieces(nres, res_off, tgt_atoms, &nfb, &lane_lds);
+    by_lane = runs.size() <= 65535;
+    if (by_lane) pieces.swap(runs);
+  }
   // Table blob (16-byte aligned sections).
   const size_t o_off = 0;
   const size_t o_tgt = round_up(o_off + sizeof(int32_t) * (nres + 1), 16);
@@ -939,11 +1010,13 @@ int rmsd_perres_nofit(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frame
   a.tvec = modify != RMSD_MODIFY_NONE ? tvec : nullptr;
   a.modify = modify == RMSD_MODIFY_ROT_TRANS ? 1 : (modify == RMSD_MODIFY_TRANS ? 2 : 0);
   a.pieces = (const int4*)(dtab + o_pc);
+  a.nfb = nfb;
   a.out = out;
   ctx->marks = 0;
   mark(ctx, 0);
   mark(ctx, 1);
-  HIP_TRY(ctx, rmsd_launch_perres(a, (int)pieces.size(), ctx->stream));
+  HIP_TRY(ctx, by_lane ? rmsd_launch_perres_lane(a, (int)pieces.size(), lane_lds, ctx->stream)
+                       : rmsd_launch_perres(a, (int)pieces.size(), ctx->stream));
   mark(ctx, 2);
   mark(ctx, 3);
   return RMSD_OK;

@@ -24,13 +24,14 @@
 // Bound by HBM (12 B per atom and frame), then by the steps' barriers: 50,000
 // AoS frames x 3,000 atoms, 194 residues of 7 to 24, masses and update, 1160 ->
 // 545 us (3.3 TB/s); centred, 20,000 x 3,000 in residues of 15, 565 -> 282 us
-// with the update and 382 -> 217 without.  The former kernel staged whole frames
-// in LDS by 4-byte transfers and gave a lane a (frame, residue): 1.5 waves per
-// SIMD, and lanes idle where residues are shorter than their wave's longest, so
-// that residues of 700 atoms took 1264 us where these take 44.  Workgroups of one
+// with the update and 382 -> 217 without.  One lane per (frame, residue) over frames
+// staged in LDS (k_perres_lane.hip) has 1.5 waves per SIMD here, and lanes idle where
+// residues are shorter than their wave's longest, so that residues of 700 atoms
+// took 1264 us where these take 44.  Workgroups of one
 // wave (pieces of 64 atoms, no barriers) give 175 us where 256 threads give 159.
-// Centred residues of fewer than 5 atoms are the ones that lose (0.54 to 0.98 of
-// the former speed: two steps and three divides for so few terms).
+// Tables of few atoms, and centred residues of fewer than 5, are the ones that
+// lose (idle threads; two steps and three divides for so few terms): those go to
+// k_perres_lane.hip, the former kernel.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include "rmsd_kernels.hpp"

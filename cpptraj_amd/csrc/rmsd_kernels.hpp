@@ -349,6 +349,7 @@ struct PerresArgs {
   const double* tvec;     // 6 per frame (modify 1, 2)
   int modify;             // 0: frames as stored; 1: x' = U (x + t) + r; 2: x + (t + r)
   const int4* pieces;
+  int nfb = 0;            // k_perres_lane: frames per batch
   double* out;            // out[f * nres + r]
 };
 constexpr int PERRES_THREADS = 256;
@@ -356,10 +357,48 @@ constexpr int PERRES_ENTRIES = 256;   // atoms of a piece
 constexpr int PERRES_RES_PIECE = 128;  // residues of a piece
 constexpr int PERRES_RES_CENTER = 64;  // ... when centred: with their centres in LDS 5
                                        // workgroups to a CU (320 us) instead of 4 (368)
-// The largest residue accepted: this many bytes by rmsd_perres_residue_bytes.
+// The largest residue accepted, this many bytes by rmsd_perres_residue_bytes: a
+// limit of the interface (once a residue's image in LDS), not of the kernels, which
+// take longer residues in stretches.
 constexpr size_t PERRES_RESIDUE_MAX = size_t(160) << 10;
 size_t rmsd_perres_residue_bytes(int natoms, int span);
 hipError_t rmsd_launch_perres(const PerresArgs& a, int npieces, hipStream_t s);
+
+// The form for small tables (k_perres_lane.hip).  pieces: {first residue, end
+// residue, lowest target atom, highest target atom + 1}, or {first, end, -1, -1}
+// for a piece that gathers its own atoms.
+constexpr int PERRES_LANE_THREADS = 64;
+constexpr int PERRES_LANE_RESIDUES = 16;                // residues of a piece
+constexpr int PERRES_LANE_MOST = 32;                    // atoms of a residue
+constexpr size_t PERRES_LANE_PIECE = size_t(12) << 10;  // LDS bytes of a piece and one frame
+constexpr size_t PERRES_LANE_BATCH = size_t(24) << 10;  // ... and a batch of frames
+constexpr size_t PERRES_LANE_LDS = size_t(64) << 10;
+size_t rmsd_perres_lane_bytes(int nres_piece, int nentries, int span, int nfb);
+hipError_t rmsd_launch_perres_lane(const PerresArgs& a, int npieces, size_t lds_bytes, hipStream_t s);
+
+// Whether a table of nres residues, `atoms` atoms in all, `most` in one and within
+// a span of target atoms, which k_perres would take in npieces pieces, goes to
+// k_perres_lane.  k_perres costs about the same for a piece of few atoms as for a
+// full one; k_perres_lane costs per atom, by its waves' longest residues, and per
+// residue, which weighs least beside centred sums (modify: 0 as stored, 1 rotated,
+// 2 translated).  Time of k_perres / k_perres_lane at 5 to 8 million residue sums:
+// centred 10 residues of 8 atoms 1.4, of 12 1.05, 15 0.75; 40 of 4 1.25, 5 1.05, 6
+// 0.85; 300 of 2 1.5, 4 1.07, 5 1.0, 6 0.92; rotated 10 of 8 1.27, 12 0.98; 40 of 3
+// 1.16, 5 1.0; 300 of 2 0.78, 4 1.08; translated 10 of 5 1.75, 8 1.12; as stored 10
+// of 6 1.07, 7 0.89; 20 of 2 1.03, 3 0.89; one residue of 30 / 60 atoms, centred
+// 1.8 / 0.8.  Where a mask leaves gaps k_perres reads only its atoms: C-alpha of 300
+// residues of 15 atoms 0.57.
+inline bool rmsd_perres_by_lane(bool center, int modify, int npieces, int nres, int atoms, int most,
+                                int span) {
+  if (most > PERRES_LANE_MOST) return false;
+  const double p = npieces, n = nres, work = 0.75 * atoms + 0.25 * n * most, gap = span - 2.0 * atoms;
+  auto upto = [&](double k) { return n < k * p ? n : k * p; };
+  if (center) return gap <= 128 && work < 71 * p + 3.5 * n;
+  if (modify == 1)
+    return gap <= 64 && (work < 75 * p + 3 * upto(12) || (work >= 2.5 * n && work < 4.2 * n));
+  if (modify == 2) return gap <= 64 && work < 70 * p + 1.5 * upto(20);
+  return span <= atoms + 32 && work < 35 * p + 2.5 * upto(10);
+}
 
 // RMS average correlation (k_avgcorr.hip): one wavefront per window size.
 struct AvgCorrArgs {

@@ -4,7 +4,7 @@ The kernel sums atom by atom in the reference's order with FP64 contraction
 off, so it agrees with the oracle to rounding of the final square root at
 most; the bar is 1e-12 A.  Cases: ragged and scattered residues, residues
 larger than a wavefront, a residue that needs a workgroup piece of its own,
-tables cut into many pieces, masses, centring, the fit's coordinate update
+tables cut into many pieces, small tables (one lane per frame and residue), masses, centring, the fit's coordinate update
 (rotate + translate, translate only), SoA frames, frame lists, a reference
 frame taken from another set, zero total mass, and argument errors.
 """
@@ -95,7 +95,7 @@ def test_perres_many_pieces_and_frames(ctx, oracle):
 
 def test_perres_oversized_residue(ctx, oracle):
     # One 3,000-atom residue (its LDS image exceeds a shared piece) between
-    # small ones; a 5,000-atom residue is beyond one workgroup and rejected.
+    # small ones; a 5,000-atom residue is past the call's limit and rejected.
     # The scattered residue of the other tests is gathered, not spanned.
     import torch
 
@@ -206,3 +206,46 @@ def test_perres_piece_edges(ctx, oracle, center, soa, F):
                          U=torch.as_tensor(U).cuda(), tvec=torch.as_tensor(tv).cuda(), soa=soa,
                          natom=n if soa else None, ctx=ctx).cpu().numpy()
     assert np.abs(got - exp).max() <= TOL
+
+
+@pytest.mark.parametrize("modify", [0, 1, 2])
+@pytest.mark.parametrize("center", [False, True])
+@pytest.mark.parametrize("nres,size,gap", [(1, 1, 0), (1, 30, 0), (1, 32, 0), (1, 33, 0), (3, 20, 0),
+                                           (6, 0, 0), (10, 5, 0), (10, 8, 0), (10, 13, 0), (17, 4, 0),
+                                           (40, 5, 0), (300, 4, 0), (300, 1, 0), (8, 1, 14), (20, 1, 14),
+                                           (7, 4, 12), (9, 3, 200)])
+def test_perres_small_tables(ctx, oracle, nres, size, gap, center, modify):
+    """Tables on both sides of the line between a lane per residue and a thread
+    per atom: few residues or centred ones of few atoms, masks with gaps (staged
+    as a span or gathered), sizes 0 to 9 mixed (size 0), frames that fill no
+    batch, AoS and SoA."""
+    import torch
+
+    import cpptraj_amd as ca
+    sizes = [(5 * i) % 10 for i in range(nres)] if size == 0 else [size] * nres
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    atoms = np.concatenate([o + i * gap + np.arange(s) for i, (o, s) in enumerate(zip(off, sizes))])
+    atoms = atoms.astype(np.int32)[::-1].copy() if nres == 17 else atoms.astype(np.int32)
+    n = int(atoms.max()) + 3
+    for F in (1, 67, 300):
+        rng = np.random.default_rng(F + nres)
+        X = synth.noisy(F + nres, F, n, 0.6).reshape(F, -1).astype(np.float32)
+        ref = (X[0] + rng.normal(size=3 * n)).astype(np.float32)
+        m = synth.masses(rng, n)
+        U = synth.rotations(rng, F).reshape(F, 3, 3)
+        tv = rng.uniform(-15, 15, size=(F, 6))
+        um = F != 67
+        exp = oracle.perres(X, ref, off, atoms, tmass=m[atoms] if um else None, use_mass=um,
+                            center=center, U=U if modify == 1 else None,
+                            tvec=tv if modify else None, modify=modify)
+        kw = dict(tmass=m[atoms] if um else None, use_mass=um, center=center,
+                  modify=("nomod", "rottrans", "norotate")[modify], ctx=ctx,
+                  U=torch.as_tensor(U).cuda() if modify == 1 else None,
+                  tvec=torch.as_tensor(tv).cuda() if modify else None)
+        R = ref.reshape(1, n, 3)
+        got = _gpu(X, ref, off, atoms, **kw)
+        assert np.abs(got - exp).max() <= TOL
+        soa = ca.rmsd_perres(torch.as_tensor(synth.to_soa(X.reshape(F, n, 3), ld=n + 1)).cuda(), off,
+                             atoms, ref_frames=torch.as_tensor(synth.to_soa(R, ld=n + 1)).cuda(),
+                             soa=True, natom=n, **kw)
+        assert np.array_equal(soa.cpu().numpy(), got)
