@@ -393,8 +393,19 @@ __device__ __forceinline__ double ac_fit(double d2, const double* ri, const doub
   return rmsd_dev::qcp_rmsd(R, 0.5 * (sx + K[3]), W, 1);
 }
 
-// Sums of a tile's RMSDs rr[64][AC_LD] along its diagonals: thread dd + 63
-// takes local diagonal dd = il - jl.
+// Fits on local diagonal dd = il - jl of row tile ti: il0 ... il1 - 1.
+__device__ __forceinline__ void ac_span(int64_t nrow, int ti, int dd, int& il0, int& il1) {
+  const int64_t rows = nrow - (int64_t)ti * AC_TILE;
+  il0 = dd > 0 ? dd : 0;
+  il1 = dd < 0 ? AC_TILE + dd : AC_TILE;
+  if (il1 > rows) il1 = (int)rows;
+}
+
+// A tile's RMSDs rr[64][AC_LD] along its diagonals, thread dd + 63 taking local
+// diagonal dd: their sum, and their squared deviations from its mean, by way of
+// the first RMSD (the mean square less the squared mean leaves the last windows,
+// whose few fits hardly differ, up to sqrt(eps) of the RMSD: 10,000 x 300, over
+// all windows, 7e-10 of the SDs' norm; so 1e-11).
 __device__ __forceinline__ void ac_diagonals(const AvgPrefixArgs& a, const double* rr, int ti,
                                              int tj) {
   const int64_t i0 = (int64_t)ti * AC_TILE, j0 = (int64_t)tj * AC_TILE;
@@ -405,11 +416,18 @@ __device__ __forceinline__ void ac_diagonals(const AvgPrefixArgs& a, const doubl
   const int64_t w = (i0 - j0) + dd;
   if (!(w >= 1 && w < nrow && a.wmap[w] >= 0)) return;
   double s1 = 0.0, s2 = 0.0;
-  const int il0 = dd > 0 ? dd : 0, il1 = dd < 0 ? AC_TILE + dd : AC_TILE;
-  for (int il = il0; il < il1; ++il) {
-    const double r = rr[il * AC_LD + il - dd];
-    s1 += r;
-    s2 += r * r;
+  int il0, il1;
+  ac_span(nrow, ti, dd, il0, il1);
+  if (il1 > il0) {
+    const double r0 = rr[il0 * AC_LD + il0 - dd];
+    double t1 = 0.0;
+    for (int il = il0; il < il1; ++il) {
+      const double r = rr[il * AC_LD + il - dd], e = r - r0;
+      s1 += r;
+      t1 += e;
+      s2 += e * e;
+    }
+    s2 -= t1 * t1 / (double)(il1 - il0);
   }
   // Slot of this tile among the two j tiles that diagonal w crosses in row
   // tile ti.
@@ -534,7 +552,7 @@ __device__ __forceinline__ void ac_direct(const AvgPrefixArgs& a, int ti, int tj
 // and, after it, the fits' vector FP64.  Tiles come in bands of eight row
 // tiles, an XCD's workgroups in one run of that order, so that tiles running
 // side by side share rows in its L2.  10,000 frames x 300 atoms, all windows: the
-// whole call 2.43 ms against 4.80 with every tile's distances from the
+// whole call 2.44 ms against 4.80 with every tile's distances from the
 // differences; MFMA pipes 54 % busy and vector issue 27 % at 2.1 GHz, three waves
 // per SIMD (four spill: 3.36 ms).  The tiles near the diagonal run in the same
 // launch: 314 of 12,400.
@@ -670,28 +688,40 @@ __global__ __launch_bounds__(AC_THREADS) __attribute__((amdgpu_waves_per_eu(3)))
 __global__ __launch_bounds__(64) void k_ac_final(AvgPrefixArgs a) {
   const int wi = blockIdx.x;
   const int w = a.windows[wi];
+  auto slots = [&](auto&& use) {
+    for (int slot = threadIdx.x; slot < 2 * a.ntile; slot += 64) {
+      const int ti = slot >> 1, half = slot & 1;
+      // The tile (ti, tj) that holds this slot; written when it exists and
+      // diagonal w crosses it (a multiple of 64 crosses one tile per row tile).
+      const int T = a.tile;
+      const int tj = ti - (w + T - 1) / T + half;
+      if (tj < 0 || tj > ti) continue;
+      const int off = w - T * (ti - tj);
+      if (off < 1 - T || off > T - 1) continue;
+      use(ti, off, a.part + (((int64_t)wi * a.ntile + ti) * 2 + half) * 2);
+    }
+  };
+  const double d = 1.0 / ((double)a.fs.nframes - (double)w + 1.0);
   double s1 = 0.0, s2 = 0.0;
-  for (int slot = threadIdx.x; slot < 2 * a.ntile; slot += 64) {
-    const int ti = slot >> 1, half = slot & 1;
-    // The tile (ti, tj) that holds this slot; written when it exists and
-    // diagonal w crosses it (a multiple of 64 crosses one tile per row tile).
-    const int T = a.tile;
-    const int tj = ti - (w + T - 1) / T + half;
-    if (tj < 0 || tj > ti) continue;
-    const int off = w - T * (ti - tj);
-    if (off < 1 - T || off > T - 1) continue;
-    const double* o = a.part + (((int64_t)wi * a.ntile + ti) * 2 + half) * 2;
+  slots([&](int, int, const double* o) {
     s1 += o[0];
     s2 += o[1];
-  }
-  s1 = rmsd_dev::wave_sum(s1);
+  });
+  const double avg = rmsd_dev::wave_sum(s1) * d;
+  // Fixed reference: the slots' own deviations and those of their means; 'first'
+  // has sums of squares.
+  if (!a.yref)
+    slots([&](int ti, int off, const double* o) {
+      int il0, il1;
+      ac_span(a.fs.nframes + 1, ti, off, il0, il1);
+      if (il1 <= il0) return;
+      const double e = o[0] / (double)(il1 - il0) - avg;
+      s2 += (double)(il1 - il0) * e * e;
+    });
   s2 = rmsd_dev::wave_sum(s2);
   if (threadIdx.x == 0) {
-    const double dw = (double)w;
-    const double d = 1.0 / ((double)a.fs.nframes - dw + 1.0);
-    const double avg = s1 * d;
     double sd = s2 * d;
-    sd -= avg * avg;
+    if (a.yref) sd -= avg * avg;
     a.ct[wi] = avg;
     a.sd[wi] = sd > 0.0 ? sqrt(sd) : 0.0;
   }

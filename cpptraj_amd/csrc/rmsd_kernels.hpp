@@ -435,7 +435,7 @@ struct AvgPrefixArgs {
   int ngram = 0;          // fixed reference: the last ngram tiles are two or more
   int gram_per_xcd = 0;   // tiles off the diagonal (tile.x - tile.y >= 2); ngram / XCDs, up
   int ntile;              // row tiles: ceil((F+1) / 64)
-  double* part;           // [nwin][ntile][2][2] per-tile sums of RMSD and RMSD^2
+  double* part;           // [nwin][ntile][2][2] per-tile sums of RMSD and its square ('first') or deviations
   int tile;               // frames per tile side (64 fixed reference, 32 'first')
   double* yref;           // 'first': [nwin][k] sqrt(m) y_w per window, else null
   double* wconst;         // 'first': [nwin][13] sum m y_w, sum m |y_w|^2, sum m mu y_w^T

@@ -222,16 +222,17 @@ def test_avgcorr_gram_tile_edges(ctx, F, n, use_mass, offset):
     assert float((sd ** 2 - sd2 ** 2)[far].abs().max()) <= 1e-12 * float(ct2.max()) ** 2
 
 
-def _exact_means(X, ref, windows):
-    """Mean RMSD per window in extended precision, and 64 eps E0 / (W r) (64
-    roundings of E0 in the FP64 solve) averaged over each window's fits."""
+def _exact_windows(X, ref, windows):
+    """Mean and SD of each window's RMSDs in extended precision, and the mean and
+    the root mean square over its fits of 64 eps E0 / (W r) (64 roundings of E0 in
+    the FP64 solve)."""
     L = np.longdouble
     F, n = X.shape[:2]
     X = X.astype(L)
     P = np.concatenate([np.zeros((1, n, 3), L), np.cumsum(X, 0)])
     y = ref.astype(L) - ref.astype(L).mean(0)
     gy = (y * y).sum()
-    mean, tol = [], []
+    out = []
     for w in windows:
         a = (P[w:] - P[:-w]) / w
         a = a - a.mean(1, keepdims=True)
@@ -244,19 +245,21 @@ def _exact_means(X, ref, windows):
         for _ in range(60):
             lam = lam - (((lam * lam + c2) * lam + c1) * lam + c0) / (4 * lam ** 3 + 2 * c2 * lam + c1)
         r = np.sqrt(2 * (E0 - lam) / n)
-        mean.append(r.mean())
-        tol.append((64 * np.finfo(float).eps * E0 / (n * r)).mean())
-    return np.array(mean, float), np.array(tol, float)
+        tol = 64 * np.finfo(float).eps * E0 / (n * r)
+        out.append([r.mean(), np.sqrt(((r - r.mean()) ** 2).mean()), tol.mean(),
+                    np.sqrt((tol ** 2).mean())])
+    return np.array(out, float).T
 
 
-@pytest.mark.parametrize("motion", ["none", "diffusing", "jumping", "breathing 3", "breathing 10"])
+@pytest.mark.parametrize("motion", ["none", "still", "diffusing", "jumping", "breathing 3", "breathing 10"])
 def test_avgcorr_large_motions(ctx, motion):
     """Trajectories whose prefix sums are large against their differences: common
     translations of 8,192 A, and internal motion of up to ten times the
     reference's size with a period of 65 frames (10: tiles that leave the product
     for the differences).  Coordinates are multiples of 2^-10 A, 256 frames and
     16 atoms: prefix sums, means and centroids are exact in FP64, what is left is
-    the solve's rounding."""
+    the solve's rounding.  Neither the mean nor the SD of a window's RMSDs (also
+    where two fits hardly differ) can be further off than the fits are."""
     import torch
 
     import cpptraj_amd as ca
@@ -271,12 +274,15 @@ def test_avgcorr_large_motions(ctx, motion):
         X += np.cumsum(np.round(rng.normal(scale=50.0, size=(F, 1, 3))), 0)
     elif motion == "jumping":
         X += np.where(f % 65 < 32, 8192.0, -8192.0)
+    elif motion == "still":
+        X = np.repeat(X[:1], F, 0)
     elif motion != "none":
         X *= 1 + float(motion.split()[1]) * np.sin(2 * np.pi * f / 65)
     X = (np.round(X * 1024) / 1024).astype(np.float32)
     assert np.array_equal(X.astype(np.float64) * 1024, np.round(X.astype(np.float64) * 1024))
     ref = (np.round((chain + rng.normal(scale=0.3, size=(n, 3))) * 1024) / 1024).astype(np.float32)
-    w, ct, _ = _avgcorr(ca, ctx, torch.as_tensor(X.reshape(F, -1)).cuda(),
-                        ref_frames=torch.as_tensor(ref.reshape(1, -1)).cuda(), method="prefix")
-    exp, tol = _exact_means(X, ref, w)
-    assert np.all(np.abs(ct.cpu().numpy() - exp) <= tol)
+    w, ct, sd = _avgcorr(ca, ctx, torch.as_tensor(X.reshape(F, -1)).cuda(),
+                         ref_frames=torch.as_tensor(ref.reshape(1, -1)).cuda(), method="prefix")
+    mean, dev, tol, tol_rms = _exact_windows(X, ref, w)
+    assert np.all(np.abs(ct.cpu().numpy() - mean) <= tol)
+    assert np.all(np.abs(sd.cpu().numpy() - dev) <= tol_rms)
