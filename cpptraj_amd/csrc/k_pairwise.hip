@@ -831,9 +831,10 @@ __global__ void k_fill_int(int* p, int n, int v) {
 }  // namespace
 
 // ---------------------------------------------------------------------------
-// Launchers.  Tile shapes: FP64 waves own 16x32 pairs (72 FP64 accumulators),
-// (16x16 in the single-matrix kernel), FP32 and split-BF16 waves 32x48 pairs (216
-// FP32 accumulators); a workgroup covers 64 x 64 (FP64) or 64 x 96 frame pairs.
+// Launchers.  Tile shapes: FP64 waves own 16 x 16 pairs (36 FP64 accumulators) in
+// the single-matrix kernel and 16 x 32 (72) in the batched ones, FP32 waves 32 x 48
+// (216 FP32 accumulators), split-BF16 waves 32 x 32 of operands shared through LDS;
+// a tile covers 64 x 64 frame pairs, in FP32 64 x 96.
 template <int PREC, int WR, int WC, int NWR, int NWC>
 static hipError_t launch_tiles(const PairArgs& a, hipStream_t s) {
   const int nblocks = a.per_xcd * a.nxcd;
@@ -869,10 +870,11 @@ static hipError_t launch_shared(const PairArgs& a, hipStream_t s) {
 }
 
 // Four waves to a workgroup while there are few blocks per SIMD: a workgroup's
-// waves go to the four SIMDs of a CU, where single waves were seen to share a
-// SIMD beside idle ones (1,024 blocks of 2,000 atoms on 1,024 SIMDs: 302 us
-// against 172).  One wave beyond (1 to 2 % faster: nothing waits for a
-// workgroup's last wave).
+// waves go to the four SIMDs of a CU, where single waves can share a SIMD beside
+// idle ones (in one session 1,024 blocks of 2,000 atoms on 1,024 SIMDs took 302 us
+// against 172; in another the two were level, as they are within 1 % from 40 to
+// 2,000 frames of 66 to 2,000 atoms).  One wave beyond: nothing waits for a
+// workgroup's last wave (1 to 3 % faster from 3,001 frames on).
 constexpr int F64_QUAD_TILES = 1024;
 template <int NW>
 static hipError_t launch_f64(const PairArgs& a, hipStream_t s) {

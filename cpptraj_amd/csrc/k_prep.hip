@@ -28,8 +28,9 @@ namespace {
 
 constexpr int PREP_THREADS = 64;
 // FP64: few frames, or fewer than a chip's fill of larger ones, take four waves
-// each (512 x 2,000: 42 -> 20 us; 101 x 66 1.3 us faster, 1,500 x 66 2.7 us slower
-// than single waves).
+// each (512 x 2,000: 42 -> 20 us for the kernel).  A whole matrix with single waves
+// against four, 30 to 2,000 atoms: 40 to 300 frames 1.04 to 1.08, 512 1.03 to 1.08,
+// 1,000 0.98 to 1.03, 2,048 1.00 to 1.01, from 3,001 0.99 to 1.01.
 constexpr bool prep_wide(int frames, int atoms) {
   return frames <= 512 || (frames < 8192 && atoms > 256);
 }

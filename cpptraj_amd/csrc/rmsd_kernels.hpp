@@ -280,7 +280,12 @@ inline bool rmsd_fit_single(int n, bool soa, bool held) {
   if (!soa) return n <= 64;
   return n <= 104 || (n <= 128 && n % 4 != 0);
 }
-constexpr int FIT_MANY_FRAMES = 16384;  // from here a wave takes several small frames
+// From here a wave takes several small frames.  One frame a wave against several, in
+// time, 4,096 / 8,192 / 12,000 / 16,384 / 100,000 frames: rotated 20 atoms 0.75 0.94
+// 0.94 1.10 1.00, 100 atoms 0.87 1.05 1.12 1.02 1.03, 256 atoms 0.96 0.99 1.06 1.03
+// 1.06; FP32 gradient 20 atoms 0.72 0.94 0.93 1.09 1.21, 128 atoms 0.87 1.02 1.07
+// 1.17 1.11, 256 atoms 0.94 0.95 0.99 0.95 0.89.
+constexpr int FIT_MANY_FRAMES = 16384;
 constexpr int FIT_FUSED_FRAMES = 1024;  // without update: more frames take the moment kernels
 constexpr int64_t FIT_GRAD64_ATOMS = 9 << 18;  // FP64 gradient: atoms of all frames, beyond quads
 constexpr int FIT_INREF_FRAMES = 512;   // more frames: the reference is prepared once, before
