@@ -185,10 +185,11 @@ def test_triangle_past_2_31_elements(oracle, ctx, precision):
 
 @pytest.mark.parametrize("F", [2, 15, 16, 17, 33, 63, 64, 65, 130])
 @pytest.mark.parametrize("n,use_mass", [(3, False), (8, True), (61, False), (515, True)])
-def test_fp64_block_edges(ctx, F, n, use_mass):
+def test_fp64_block_edges(oracle, ctx, F, n, use_mass):
     """The FP64 matrix in 16 x 16 blocks at the edges of blocks and tiles and of
-    the weight sum's stages: the triangle has the batched kernel's bits, the
-    full matrix of its first frames against all the triangle's values."""
+    the weight sum's stages: the triangle against the oracle and with the batched
+    kernel's bits, the full matrix of its first frames against all the triangle's
+    values."""
     import torch
     import cpptraj_amd as ca
     X = torch.as_tensor(synth.noisy(F + n, F, n, 0.7).reshape(F, -1)).cuda()
@@ -196,6 +197,10 @@ def test_fp64_block_edges(ctx, F, n, use_mass):
     tri = ca.rms2d(X, mass=m, use_mass=use_mass, ctx=ctx)
     bat = ca.rms2d_batch([X], masses=[m], use_mass=use_mass, precision="fp64", ctx=ctx)[0]
     assert torch.equal(tri, bat)
+    # Three atoms, a plane: the oracle's QCP (its Kabsch eigenvalues are 1e-6 A off).
+    exp = oracle.rms2d(X.cpu().numpy(), None, m.cpu().numpy(), MODE["qrmsd" if n == 3 else "fit"],
+                       use_mass)
+    assert np.abs(tri.cpu().numpy().astype(np.float64) - exp).max() <= 1e-6
     k = max(1, F // 2)
     full = ca.rms2d(X[:k], mass=m, use_mass=use_mass, ref_frames=X, ref_mass=m, ctx=ctx)
     iu = torch.triu_indices(F, F, 1, device="cuda")
