@@ -946,7 +946,7 @@ int rmsd_perres_nofit(rmsd_ctx* ctx, const rmsd_frames* frames, const rmsd_frame
   auto by_lane_for = [&](int span) {
     return rmsd_perres_by_lane(
         center != 0, modify == RMSD_MODIFY_ROT_TRANS ? 1 : (modify == RMSD_MODIFY_TRANS ? 2 : 0),
-        (int)pieces.size(), nres, L, most, span);
+        frames->ld != 0, frames->nframes, (int)pieces.size(), nres, L, most, span);
   };
   bool by_lane = by_lane_for(0);
   if (by_lane && L) {  // the span of the atoms only where it can matter

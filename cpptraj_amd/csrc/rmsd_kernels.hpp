@@ -389,19 +389,22 @@ hipError_t rmsd_launch_perres_lane(const PerresArgs& a, int npieces, size_t lds_
 // 2 translated).  Time of k_perres / k_perres_lane at 5 to 8 million residue sums:
 // centred 10 residues of 8 atoms 1.4, of 12 1.05, 15 0.75; 40 of 4 1.25, 5 1.05, 6
 // 0.85; 300 of 2 1.5, 4 1.07, 5 1.0, 6 0.92; rotated 10 of 8 1.27, 12 0.98; 40 of 3
-// 1.16, 5 1.0; 300 of 2 0.78, 4 1.08; translated 10 of 5 1.75, 8 1.12; as stored 10
-// of 6 1.07, 7 0.89; 20 of 2 1.03, 3 0.89; one residue of 30 / 60 atoms, centred
-// 1.8 / 0.8.  Where a mask leaves gaps k_perres reads only its atoms: C-alpha of 300
-// residues of 15 atoms 0.57.
-inline bool rmsd_perres_by_lane(bool center, int modify, int npieces, int nres, int atoms, int most,
-                                int span) {
-  if (most > PERRES_LANE_MOST) return false;
+// 1.16, 5 1.0; 300 of 1 0.76 (50,000 frames), 4 0.93; translated 10 of 5 1.75, 8
+// 1.12; as stored 10 of 6 1.07, 7 0.89; 20 of 2 1.03, 3 0.89 (SoA: 1 of 8 0.86, 10
+// of 5 1.12, 40 of 1 0.79); one residue of 30 / 60 atoms, centred 1.8 / 0.8.  Where a
+// mask leaves gaps k_perres reads only its atoms: C-alpha of 300 residues of 15 atoms
+// 0.57.  A large table in a short call is bound by the host, which cuts
+// k_perres_lane's pieces more slowly (300 x 3,000, 4 atoms each, 28.7 us against
+// 33.5).
+inline bool rmsd_perres_by_lane(bool center, int modify, bool soa, int64_t nframes, int npieces,
+                                int nres, int atoms, int most, int span) {
+  if (most > PERRES_LANE_MOST || (atoms > 512 && nframes * atoms < 2000000)) return false;
   const double p = npieces, n = nres, work = 0.75 * atoms + 0.25 * n * most, gap = span - 2.0 * atoms;
   auto upto = [&](double k) { return n < k * p ? n : k * p; };
-  if (center) return gap <= 128 && work < 71 * p + 3.5 * n;
-  if (modify == 1)
-    return gap <= 64 && (work < 75 * p + 3 * upto(12) || (work >= 2.5 * n && work < 4.2 * n));
+  if (center) return gap <= 128 && work < 71 * p + (soa ? 3.0 : 3.5) * n;
+  if (modify == 1) return gap <= 64 && n <= 48 * p && work < 75 * p + 3 * upto(12);
   if (modify == 2) return gap <= 64 && work < 70 * p + 1.5 * upto(20);
+  if (soa && (n < 3 || n > 16 * p)) return false;
   return span <= atoms + 32 && work < 35 * p + 2.5 * upto(10);
 }
 
