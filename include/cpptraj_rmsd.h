@@ -101,9 +101,9 @@ int64_t rmsd_ctx_scratch_bytes(const rmsd_ctx* ctx);
 
 /* Stage timing (the counterpart of cpptraj's Timer around an analysis,
  * src/Timer.h:10-20, at kernel granularity).  With profiling on, every call but
- * rmsd_fit_to_ref_noalloc (which may be captured)
- * records HIP events on the context's stream; rmsd_ctx_stage_ms waits for the
- * last call and returns three durations in milliseconds:
+ * rmsd_fit_to_ref_noalloc (which may be captured) records HIP events on the
+ * context's stream; rmsd_ctx_stage_ms waits for the last such call and returns
+ * three durations in milliseconds:
  *   ms[0] per-frame stage (setup, gather/centre/pack; reference preparation),
  *   ms[1] the main kernel (pair contraction + QCP; streaming moments),
  *   ms[2] per-frame epilogue (fit solve / coordinate update; 0 for pairwise). */
